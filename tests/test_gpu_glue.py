@@ -203,3 +203,57 @@ def test_attention_prefill(lib, nh, nkv, hd, max_seq, m, pos0, order):
     out2 = torch.full_like(out, float("nan"))
     run(out2)
     assert torch.equal(out[vr], out2[vr])
+
+
+@pytest.mark.parametrize("nh,nkv,hd,max_seq,m,pos0", [
+    (4, 4, 64, 65, 1, 64),        # one row past a key tile
+    (2, 1, 128, 64, 31, 33),      # a 32-row block less one, the last slot
+    (4, 1, 128, 300, 33, 63),     # a row past a block; tile edges inside the rows
+    (3, 1, 128, 200, 65, 0),      # heads and row blocks mixed in a workgroup
+    (2, 2, 256, 130, 32, 96),     # 32-key tiles
+    (1, 1, 256, 40, 17, 0),       # the second query pass holds one row
+])
+@pytest.mark.parametrize("scale", ["plain", "mixed"])
+def test_attention_prefill_edges(lib, nh, nkv, hd, max_seq, m, pos0, scale):
+    """Tile and block edges, and operands of mixed magnitude: with "mixed" the keys
+    and values of each 4 slots carry a power of two of their own in 2^-12 .. 2^12
+    and the queries 2^-8, and a key no row sees is infinite.
+
+    Bound, with u = 2^-24: an operand's hi + lo parts hold it to 2 u and the dropped
+    lo lo product is below 4 u of its term, so a score is within 16 u sum |q k| and
+    the f32 sums of it and of hd (RoPE included) products add less than that again;
+    a probability moves by its score's error, and the sum of p v by its own.  In
+    ratio to sum p |v|: 64 u (1 + max sum |q k| / sqrt(hd))."""
+    g = torch.Generator(device="cuda").manual_seed(hd + m)
+    row, orow, grp, half = (nh + 2 * nkv) * hd, nh * hd, nh // nkv, hd // 2
+    qkv = torch.randn(m, row, device="cuda", generator=g)
+    kc = torch.randn(nkv, max_seq, hd, device="cuda", generator=g)
+    vc = torch.randn(nkv, max_seq, hd, device="cuda", generator=g)
+    if scale == "mixed":
+        e = torch.randint(-12, 13, (max_seq,), device="cuda", generator=g)
+        e = torch.exp2(e[torch.arange(max_seq, device="cuda") // 4 * 4].float())[None, :, None]
+        kc, vc = kc * e, vc * e
+        qkv[:, :orow] *= 2.0 ** -8
+    if pos0 + m < max_seq:
+        kc[:, pos0 + m:] = float("inf")
+    inv, cos, sin = _rope_inv(hd, max_seq)
+    pos = torch.arange(pos0, pos0 + m, device="cuda")
+    out = torch.full((m, orow), float("nan"), device="cuda")
+    _ok(lib, lib.gguf_hip_attention_prefill(qkv.data_ptr(), row, pos.data_ptr(), m, cos.data_ptr(),
+                                            sin.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                                            out.data_ptr(), orow, nh, nkv, hd, max_seq, _s()))
+    c, s = cos[pos].double()[:, None], sin[pos].double()[:, None]
+    q = qkv[:, :orow].double().view(m, nh, hd)
+    a, b = q[..., :half], q[..., half:]
+    q = torch.cat([a * c - b * s, b * c + a * s], dim=-1)
+    t = pos0 + m
+    masked = torch.arange(t, device="cuda")[None] > pos[:, None]
+    for h in range(nh):
+        k, v = kc[h // grp, :t].double(), vc[h // grp, :t].double()
+        sc = (q[:, h] @ k.T / math.sqrt(hd)).masked_fill(masked, float("-inf"))
+        mag = (q[:, h].abs() @ k.abs().T / math.sqrt(hd)).masked_fill(masked, 0).amax(1)
+        p = torch.softmax(sc, dim=1)
+        err = (out[:, h * hd:(h + 1) * hd].double() - p @ v).abs()
+        lim = 64 * 2.0 ** -24 * (1 + mag)[:, None] * (p @ v.abs())
+        assert torch.isfinite(out[:, h * hd:(h + 1) * hd]).all()
+        assert (err <= lim).all(), (h, (err / lim).max().item())
