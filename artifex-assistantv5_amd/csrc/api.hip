@@ -380,7 +380,7 @@ int gguf_hip_attention_decode_noalloc(const float *qkv, const int64_t *pos,
                                       void *stream) {
   int rc = check_attention(n_heads, n_kv_heads, head_dim, max_seq);
   if (rc) return rc;
-  const int64_t need = gguf::attention_work_bytes(n_heads, n_kv_heads, head_dim, max_seq);
+  const int64_t need = gguf::attention_noalloc_bytes(n_heads, n_kv_heads, head_dim, max_seq);
   if (need > gguf::kNoAllocAttentionBytes)
     return fail(GGUF_HIP_ERR_SHAPE,
                 "[gguf-hip] attention_decode_noalloc: the shape needs %lld bytes of workspace, "

@@ -417,6 +417,9 @@ namespace gguf {
 //   M = max_s m_s,  w_s = exp(m_s - M),  L = sum_s w_s l_s,
 //   out = (sum_s w_s o_s) * (1 / L).
 constexpr int kAttnSplit = 64;
+// Up to kMergeChunk splits (of max_seq) the output projection merges the records
+// in its prologue; longer caches take attn_merge_kernel and the plain projection.
+constexpr int kMergeChunk = 8;
 constexpr int attn_record_stride(int hd) { return hd + 4; }
 struct AttnRecords {
   const float *work;     // the records
@@ -460,6 +463,9 @@ hipError_t launch_rmsnorm(float *x, const float *r, const float *w, float eps, f
                           int64_t rows, int64_t n, hipStream_t s);
 hipError_t launch_swiglu(const float *gu, float *out, int64_t rows, int64_t ffn, hipStream_t s);
 int64_t attention_work_bytes(int nh, int nkv, int hd, int64_t max_seq);
+int64_t attention_noalloc_bytes(int nh, int nkv, int hd, int64_t max_seq);
+// Merges the records into the workspace; *merged = the output [nh * hd].
+hipError_t launch_attn_merge(const AttnRecords &ar, const float **merged, hipStream_t s);
 hipError_t launch_attention_decode(const float *qkv, const int64_t *pos, const float *cs,
                                    const float *sn, float *kc, float *vc, float *out, float *work,
                                    int nh, int nkv, int hd, int64_t max_seq, hipStream_t s);

@@ -1065,7 +1065,6 @@ __device__ __forceinline__ void unit_compute(const Unit<23> &u, const Stage &st,
 // Activation staging.  Activations are converted in items of 16 consecutive
 // elements of one row, one item per thread and step.
 constexpr int kItem = 16;
-constexpr int kMergeChunk = 8;  // attention records per item held in registers (merge prologue)
 
 template <typename XT>
 __device__ __forceinline__ void load_item(const XT *__restrict__ x, int64_t ldx, int K, int k0,
@@ -1413,7 +1412,7 @@ int64_t mb_work_floats(int M, int N, int K) {
 //   PRO = 3  x is the attention output, merged here from the partial-softmax
 //            records that the decode attention wrote (no merge pass of its
 //            own): each thread's item is a 16-element slice of one query
-//            head, and the records of the first kMergeChunk splits are
+//            head, and its records (at most kMergeChunk splits) are
 //            requested with the activations, ahead of the weights;
 // and the epilogue `epi`:
 //   0  y = result;
@@ -1489,21 +1488,18 @@ __global__ __launch_bounds__(512) void decode_m1_kernel(const XT *__restrict__ x
     if constexpr (PRO == 1) load_item<float>(pw, 0, K, 0, per_row, per_row, q, pv[i]);
     if constexpr (PRO == 2) load_item<float>((const float *)x + K, 0, K, 0, per_row, per_row, q, pv[i]);
   }
-  // PRO 3: the item's 16-element slice of the first RC attention records of
-  // its query head (the slots past the range are not loaded and get weight
-  // zero), and where the rest would be
+  // PRO 3: the item's 16-element slice of the attention records of its query
+  // head (the slots past the range are not loaded and get weight zero)
   constexpr int RC = PRO == 3 ? kMergeChunk : 1;
   float4 ro[PRO == 3 ? XI : 1][RC][4];
   float2 rml[PRO == 3 ? XI : 1][RC];
-  const float *ro_base[PRO == 3 ? XI : 1], *rml_base[PRO == 3 ? XI : 1];
   int mn = 0;              // records to merge: ceil((p + 1) / kAttnSplit), 0 for a bad p
-  int64_t rstride = 0;     // floats from one split's record to the next
   if constexpr (PRO == 3) {
     const int64_t p = ar.pos[0];
     mn = (p >= 0 && p < ar.max_seq) ? (int)(p / kAttnSplit) + 1 : 0;
     const int grp = ar.nh / ar.nkv, S = (ar.max_seq + kAttnSplit - 1) / kAttnSplit;
     const int rs = attn_record_stride(ar.hd);
-    rstride = (int64_t)grp * rs;
+    const int64_t rstride = (int64_t)grp * rs;  // floats from one split's record to the next
     const int last = mn > 0 ? mn - 1 : 0;
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
@@ -1511,16 +1507,14 @@ __global__ __launch_bounds__(512) void decode_m1_kernel(const XT *__restrict__ x
       const int k0 = kItem * q, h = k0 / ar.hd, i0 = k0 - h * ar.hd;
       const int gk = h / grp, jh = h - gk * grp;
       const float *rec = ar.work + ((int64_t)gk * S * grp + jh) * rs;
-      ro_base[i] = rec + i0;
-      rml_base[i] = rec + ar.hd;
 #pragma unroll
       for (int c = 0; c < RC; ++c) {
         if (c > last) break;  // uniform: the loads of splits past the range are not issued
         const int64_t off = (int64_t)c * rstride;
-        const float4 *o4 = (const float4 *)(ro_base[i] + off);
+        const float4 *o4 = (const float4 *)(rec + i0 + off);
 #pragma unroll
         for (int v = 0; v < 4; ++v) ro[i][c][v] = o4[v];
-        rml[i][c] = *(const float2 *)(rml_base[i] + off);
+        rml[i][c] = *(const float2 *)(rec + ar.hd + off);
       }
     }
   }
@@ -1579,7 +1573,6 @@ __global__ __launch_bounds__(512) void decode_m1_kernel(const XT *__restrict__ x
 #pragma unroll
       for (int c = 0; c < RC; ++c)
         if (c < mn) M = fmaxf(M, rml[i][c].x);
-      for (int s2 = RC; s2 < mn; ++s2) M = fmaxf(M, rml_base[i][s2 * rstride]);
       float L = 0.f, a[kItem];
 #pragma unroll
       for (int e = 0; e < kItem; ++e) a[e] = 0.f;
@@ -1595,13 +1588,6 @@ __global__ __launch_bounds__(512) void decode_m1_kernel(const XT *__restrict__ x
           a[4 * v + 2] = fmaf(w, ro[i][c][v].z, a[4 * v + 2]);
           a[4 * v + 3] = fmaf(w, ro[i][c][v].w, a[4 * v + 3]);
         }
-      }
-      for (int s2 = RC; s2 < mn; ++s2) {  // ranges beyond RC splits: one record at a time
-        const float *rp = ro_base[i] + s2 * rstride, *ml = rml_base[i] + s2 * rstride;
-        const float w = expf(ml[0] - M);
-        L = fmaf(w, ml[1], L);
-#pragma unroll
-        for (int e = 0; e < kItem; ++e) a[e] = fmaf(w, rp[e], a[e]);
       }
       const float inv = 1.0f / L;  // no records (bad position): 0 * inf = NaN
 #pragma unroll

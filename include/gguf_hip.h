@@ -318,7 +318,9 @@ int gguf_hip_attention_prefill(const float *qkv, int64_t ldqkv, const int64_t *p
  * the reference's attention-output and o-projection dispatches
  * (forward-pass.ts:2925-3297) by one.  The shapes are those of the attention
  * call; K = n_heads * head_dim <= 8192.  A position outside 0..max_seq - 1
- * gives NaN outputs. */
+ * gives NaN outputs.  One launch up to 512 cache slots; longer caches take two,
+ * the first of which merges the records into the workspace (so work is written,
+ * the records are not). */
 int gguf_hip_matmul_attn_merge(const void *work, const int64_t *pos, int n_heads, int n_kv_heads,
                                int head_dim, int64_t max_seq, const void *tiles, int ggml_type,
                                int64_t n, float *y, int epilogue, void *stream);

@@ -152,7 +152,7 @@ def _attention_inputs(nh, nkv, hd, max_seq, p):
 
 
 # positions: one split, a full split, two splits, the register chunk of eight
-# splits exactly, and ranges past it (records merged one at a time)
+# splits exactly, and caches of more splits (a merge launch)
 @pytest.mark.parametrize("t,nh,nkv,hd,max_seq,p", [
     (12, 32, 8, 128, 1200, 0), (12, 32, 8, 128, 1200, 63), (12, 32, 8, 128, 1200, 64),
     (12, 32, 8, 128, 1200, 300), (12, 32, 8, 128, 1200, 511), (12, 32, 8, 128, 1200, 1199),
@@ -174,6 +174,15 @@ def test_attention_merge_projection(mods, t, nh, nkv, hd, max_seq, p):
 @pytest.mark.parametrize("p", [130, 511])
 def test_attention_merge_projection_n4096_small_blocks(mods, t, p):
     _merge_case(mods, t, 32, 8, 128, 600, p, 4096)
+
+
+# caches past the prologue's eight splits are merged by a launch of their own, 64
+# records at a time: nine splits, and ranges of 63, 64, 65, 128 and 130 records
+@pytest.mark.parametrize("nh,nkv,hd,max_seq,p", [
+    (8, 2, 128, 513, 512), (8, 2, 128, 576, 3), (4, 4, 64, 8300, 4031), (2, 1, 256, 8300, 4095),
+    (2, 1, 128, 8300, 4096), (4, 2, 64, 8192, 8191), (2, 1, 256, 8300, 8299)])
+def test_attention_merge_launch(mods, nh, nkv, hd, max_seq, p):
+    _merge_case(mods, 12 if nh * hd % 256 == 0 else 8, nh, nkv, hd, max_seq, p, 256)
 
 
 def _merge_case(mods, t, nh, nkv, hd, max_seq, p, n):
