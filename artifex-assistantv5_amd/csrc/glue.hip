@@ -950,7 +950,7 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float *__restrict_
 }
 
 // Workspace: the records [nkv][S][grp][hd + 4] floats, the merged output of
-// launch_attn_merge [nh][hd], then nkv counters.
+// launch_attn_merge [nh][hd] (more than kMergeChunk splits), then nkv counters.
 static int64_t attention_record_bytes(int nh, int nkv, int hd, int64_t max_seq) {
   const int64_t S = (max_seq + kSplit - 1) / kSplit;
   return (int64_t)sizeof(float) * nkv * S * (nh / nkv) * attn_record_stride(hd);
@@ -964,7 +964,8 @@ int64_t attention_noalloc_bytes(int nh, int nkv, int hd, int64_t max_seq) {
 }
 
 int64_t attention_work_bytes(int nh, int nkv, int hd, int64_t max_seq) {
-  return attention_noalloc_bytes(nh, nkv, hd, max_seq) + (int64_t)sizeof(float) * nh * hd;
+  const bool merge = (max_seq + kSplit - 1) / kSplit > kMergeChunk;  // launch_attn_merge's output
+  return attention_noalloc_bytes(nh, nkv, hd, max_seq) + (merge ? (int64_t)sizeof(float) * nh * hd : 0);
 }
 
 hipError_t launch_attn_merge(const AttnRecords &ar, const float **merged, hipStream_t s) {
