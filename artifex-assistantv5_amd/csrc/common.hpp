@@ -454,6 +454,15 @@ hipError_t launch_gemm(const void *x, int x_type, int64_t ldx, const uint8_t *ti
                        int64_t n, int64_t k, float *y, int64_t ldy, int64_t m, float *work,
                        int64_t work_floats, hipStream_t s);
 int64_t launch_gemm_work(int type, int x_type, int64_t n, int64_t k, int64_t m);
+hipError_t launch_gemm_reduce(const float *part, int sp, int M, int N, float *y, int64_t ldy,
+                              hipStream_t s);
+// The f32-grade GEMM (gemm_f32.hip) of batches past 32 f32 rows, with a workspace
+// of gemm_f32_work floats.
+bool gemm_f32_serves(int type, int x_type, int64_t n, int64_t k, int64_t m);
+int64_t gemm_f32_work(int type, int64_t n, int64_t k, int64_t m);
+hipError_t launch_gemm_f32(const float *x, int64_t ldx, const uint8_t *tiles, int type, int64_t n,
+                           int64_t k, float *y, int64_t ldy, int64_t m, float *work,
+                           hipStream_t s);
 hipError_t launch_decode_fused(const float *x, const uint8_t *tiles, int type, int64_t n,
                                int64_t k, float *y, int prologue, const float *pw, float eps,
                                int epilogue, hipStream_t s);

@@ -93,13 +93,23 @@ int64_t launch_decode_work(int type, int x_type, int64_t n, int64_t k, int64_t m
     const int64_t v = pass_work(type, x_type, (int)n, (int)k, (int)(m % 32));
     w = v > w ? v : w;
   }
+  if (gemm_f32_serves(type, x_type, n, k, m)) {
+    const int64_t v = kWsPrefix / 4 + gemm_f32_work(type, n, k, m);
+    w = v > w ? v : w;
+  }
   return w;
 }
 
-// Rows are processed in groups of at most 32 (one pass over the weights each).
+// Rows are processed in groups of at most 32 (one pass over the weights each);
+// larger f32 batches of the types it serves take the f32-grade GEMM when the
+// workspace holds its image.
 hipError_t launch_decode(const void *x, int x_type, int64_t ldx, const uint8_t *tiles, int type,
                          int64_t n, int64_t k, float *y, int64_t ldy, int64_t m, float *work,
                          int64_t work_floats, hipStream_t s) {
+  if (work && gemm_f32_serves(type, x_type, n, k, m) &&
+      work_floats >= kWsPrefix / 4 + gemm_f32_work(type, n, k, m))
+    return launch_gemm_f32((const float *)x, ldx, tiles, type, n, k, y, ldy, m,
+                           work + kWsPrefix / 4, s);
   const int esize = x_type == 0 ? 4 : 2;
   hipError_t e = hipSuccess;
   for (int64_t m0 = 0; m0 < m && e == hipSuccess; m0 += 32) {

@@ -2258,14 +2258,7 @@ hipError_t launch_type(const XT *x, int64_t ldx, const uint8_t *W, int M, int N,
                      sp > 1 ? (int64_t)N : ldy, tiles_m, kunits, rowf);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || sp == 1) return e;
-  const int64_t mn = (int64_t)M * N;
-  if (N % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0 && ((uintptr_t)work & 15) == 0)
-    hipLaunchKernelGGL(gemm_reduce4_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, s,
-                       (const float4 *)work, sp, M, N / 4, y, ldy);
-  else
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, work,
-                       sp, M, N, y, ldy);
-  return hipGetLastError();
+  return launch_gemm_reduce(work, sp, M, N, y, ldy, s);
 }
 
 template <typename XT>
@@ -2309,6 +2302,19 @@ hipError_t launch_x(const XT *x, int64_t ldx, const uint8_t *W, int type, int64_
 }
 
 }  // namespace
+
+// y = the sum of the sp partial sums [sp][M][N], in split order.
+hipError_t launch_gemm_reduce(const float *part, int sp, int M, int N, float *y, int64_t ldy,
+                              hipStream_t s) {
+  const int64_t mn = (int64_t)M * N;
+  if (N % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)y & 15) == 0 && ((uintptr_t)part & 15) == 0)
+    hipLaunchKernelGGL(gemm_reduce4_kernel, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, s,
+                       (const float4 *)part, sp, M, N / 4, y, ldy);
+  else
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, part,
+                       sp, M, N, y, ldy);
+  return hipGetLastError();
+}
 
 // Workspace floats of the GEMM for these shapes (0: none): for f32
 // activations their fp16 image (of the largest launch_gemm chunk of rows),

@@ -95,7 +95,9 @@ extern "C" {
 #define GGUF_HIP_VARIANT_DECODE 1 /* matrix-core decode: exact quant codes x f16 hi + lo
                                      parts of the activations scaled by a power of two
                                      per 256- or 32-element unit, f32 scales; one pass
-                                     over the weights per 32 activation rows (any M) */
+                                     over the weights per 32 activation rows (any M),
+                                     or, with a workspace, the f32-grade GEMM for 33 ..
+                                     511 f32 rows of Q4_K, Q5_K and Q6_K */
 #define GGUF_HIP_VARIANT_GEMM 2   /* MFMA GEMM with dequantized fp16 weight tiles and fp16
                                      activations staged in LDS (prefill); f32 activation
                                      rows are scaled by a power of two each first */

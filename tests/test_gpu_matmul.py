@@ -91,6 +91,34 @@ def test_decode_is_f32_grade(pkg, ref, t):
         assert met["finite"] and met["elemwise"] <= DECODE_TOL, ((t, m, n, k), met)
 
 
+@pytest.mark.parametrize("t", [12, 13, 14])
+@pytest.mark.parametrize("m,n,k", [
+    (33, 1, 256),       # one unit: the second K half of the workgroup is empty; one column
+    (48, 257, 768),     # an odd count of units; a column past a block
+    (64, 130, 512),     # a full row block; Q6_K's 128-column blocks
+    (65, 193, 1280),    # a row past a block; Q5_K's 192-column blocks
+    (127, 31, 4096),    # few workgroups: the K range is split over the grid
+    (200, 600, 2816),   # uneven K splits
+    (511, 40, 512),     # the largest batch
+])
+def test_f32_gemm_is_f32_grade(pkg, ref, t, m, n, k):
+    """33 .. 511 f32 rows: as test_decode_is_f32_grade, rows of mixed magnitude (each
+    256-element unit of a row carries a power of two of its own) included, and the
+    same bits from a second call."""
+    raw, w = _case(pkg, t, n, k, seed=m + n)
+    wdeq = ref.dequant_rows(t, raw, n, k)
+    x = pkg.quantize.synthetic_activations(m, k, seed=m + k)
+    e = np.random.default_rng(m).integers(-40, 41, (m, k // 256))
+    e[::2] = 0
+    x = (x * np.repeat(np.exp2(e), 256, axis=1)).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    y = pkg.qlinear(xd, w)
+    assert torch.equal(y, pkg.qlinear(xd, w))
+    x64 = x.astype(np.float64)
+    met = ref.parity_metrics(y.cpu().numpy(), ref.matmul_bt(x64, wdeq), ref.matmul_bt_abs(x64, wdeq))
+    assert met["elemwise"] <= DECODE_TOL, met
+
+
 @pytest.mark.parametrize("t", [14, 8, 12])
 @pytest.mark.parametrize("xdt", [np.float32, np.float16])
 def test_batched_decode_random_blocks(pkg, ref, t, xdt):
