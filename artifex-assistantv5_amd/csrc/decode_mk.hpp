@@ -1,4 +1,5 @@
-// Batched decode of Q4_K, Q6_K, Q8_0 and the grid-codebook IQ weights
+// Batched decode of Q4_K, Q5_K, Q6_K, the 32-element-block types (Q8_0, Q4_0, Q5_0,
+// IQ4_NL), IQ4_XS and the grid-codebook IQ weights
 // (2 <= M <= 32 activation rows, and M = 1 beyond the one-shot kernel's K).
 //
 // Replaces the reference's batched decode, which runs its Q4_K GEMV once per
@@ -32,7 +33,8 @@
 // MFMAs of a unit chain into one f32 accumulator D[m, n] = sum_j sc_j sum_k q x;
 // one 16x16x16 MFMA gives the mins' dot M[m, n] = sum_j m_j S_j[m]; then
 //     acc[m, n] += F[m] (d D[m, n] - 32 dmin M[m, n])
-// in f32, and the parts are added at the end.
+// in f32, and the parts are added at the end.  Q5_K's operand is sc (q - 16), and
+// 16 d times the scales' dot with the sums is added.
 #pragma once
 
 constexpr int kMkLd = 256 + 8;  // halves per staged row: a 16-byte pad (bank spread)
@@ -59,12 +61,17 @@ constexpr int mk_f_off() {
 //          2: as 1, and within each 32-element window the quads of its two
 //          16-element groups interleaved (Q6_K: lane group g's 8 k are quad g
 //          of group 2t, then quad g of group 2t + 1)
-//   NF     inverse scales per unit and row (Q8_0: one per block)
+//   NF     inverse scales per unit and row (the block types and IQ4_XS: one per
+//          32-element block)
+constexpr bool mk_blocks(int type) {
+  return type == 8 || type == 2 || type == 6 || type == 20 || type == 23;
+}
 template <int TYPE>
 struct MkFmt {
-  static constexpr int ORDER = TYPE == 12 ? 1 : 0, NF = 1;
-  static constexpr bool SUMS = TYPE == 12;
-  static constexpr int TU = Fmt<TYPE>::TU;  // bytes of a row tile's unit
+  static constexpr int ORDER = TYPE == 12 || TYPE == 13 || mk_blocks(TYPE) ? 1 : 0;
+  static constexpr int NF = mk_blocks(TYPE) ? 8 : 1;
+  static constexpr bool SUMS = TYPE == 12 || TYPE == 13;
+  static constexpr int TU = 256 / Fmt<TYPE>::UE * Fmt<TYPE>::TU;  // bytes of a row tile's unit
 };
 template <>
 struct MkFmt<14> {
@@ -72,33 +79,45 @@ struct MkFmt<14> {
   static constexpr bool SUMS = false;
   static constexpr int TU = Fmt<14>::TU;
 };
-template <>
-struct MkFmt<8> {
-  static constexpr int ORDER = 1, NF = 8;
-  static constexpr bool SUMS = false;
-  static constexpr int TU = 8 * Fmt<8>::TU;
-};
 template <int TYPE, int MA>
 constexpr int mk_ub() {
   return mk_unit_bytes<MA, MkFmt<TYPE>::SUMS, MkFmt<TYPE>::NF>();
 }
 
-// The weight unit a lane holds: Unit<TYPE>, or eight Q8_0 blocks.
-struct Q8Super {
-  Unit<8> b[8];
+// The weight unit a lane holds: Unit<TYPE>, or eight 32-element blocks.
+template <int TYPE>
+struct Blocks8 {
+  Unit<TYPE> b[8];
 };
 template <int TYPE>
 struct MkUnitOf {
-  using type = Unit<TYPE>;
+  using type = std::conditional_t<mk_blocks(TYPE) && TYPE != 23, Blocks8<TYPE>, Unit<TYPE>>;
 };
-template <>
-struct MkUnitOf<8> {
-  using type = Q8Super;
-};
+template <int TYPE>
 __device__ __forceinline__ void load_unit(__amdgpu_buffer_rsrc_t rs, int soff, int r, int g,
-                                          Q8Super &u) {
+                                          Blocks8<TYPE> &u) {
 #pragma unroll
-  for (int b = 0; b < 8; ++b) load_unit(rs, soff + b * Fmt<8>::TU, r, g, u.b[b]);
+  for (int b = 0; b < 8; ++b) load_unit(rs, soff + b * Fmt<TYPE>::TU, r, g, u.b[b]);
+}
+// Block b's codes for lane group g, exact signed f16 integers in quad order, and its scale
+template <int TYPE>
+__device__ __forceinline__ half8_t mk_block(const Blocks8<TYPE> &u, int b, int g) {
+  if constexpr (TYPE == 8) {
+    return q8_operand(u.b[b]);
+  } else {
+    uint32_t qhb = 0, w[4];
+    if constexpr (TYPE == 6) qhb = (u.b[b].qh >> (8 * g)) & 0xFFu;
+    b32_f16<TYPE>(u.b[b].q, qhb, w);
+    return as_h8(w[0], w[1], w[2], w[3]);
+  }
+}
+__device__ __forceinline__ half8_t mk_block(const Unit<23> &u, int b, int) { return xs_codes(u, b); }
+template <int TYPE>
+__device__ __forceinline__ float mk_block_scale(const Blocks8<TYPE> &u, int b) {
+  return h2f(u.b[b].d);
+}
+__device__ __forceinline__ float mk_block_scale(const Unit<23> &u, int b) {  // exact
+  return h2f(u.h.x) * (float)((int)iq4xs_ls(u.h.x >> 16, u.h.y, b) - 32);
 }
 
 #ifndef GGUF_MK_LDS
@@ -227,8 +246,18 @@ __device__ __forceinline__ uint32_t mk_scaled(uint32_t w, uint32_t m, uint32_t b
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(c, scp, nsp));
 }
 
-template <int MA, int T>
-__device__ __forceinline__ void mk_unit(const Unit<12> (&w)[T], int bo, int lane, bool valid,
+// Q5_K: sc (q - 16) for the same, the fifth bits in place in f (off = -1024 - 16, or
+// -1024 - 256 for high nibbles).  Around the middle of its codes the products' running
+// sum, and so its f32 rounding, is half of sc q's (3.2e-7 against float64 with sc q at
+// 12 x 14336 x 4096, 2.6e-7 the kernel before).
+__device__ __forceinline__ uint32_t mk_centred(uint32_t w, uint32_t m, uint32_t base, half2_t scp,
+                                               half2_t off, uint32_t f) {
+  const half2_t c = __builtin_bit_cast(half2_t, and_or(w, m, base) | f);
+  return __builtin_bit_cast(uint32_t, (c + off) * scp);
+}
+
+template <int TYPE, int MA, int T>
+__device__ __forceinline__ void mk_unit(const Unit<TYPE> (&w)[T], int bo, int lane, bool valid,
                                         float (&acc)[T][MA][4]) {
 #pragma clang fp contract(off)
   const int r = lane & 15, g = lane >> 4;
@@ -239,11 +268,13 @@ __device__ __forceinline__ void mk_unit(const Unit<12> (&w)[T], int bo, int lane
   // SC[t][i]: scales (sc0, sc2), (sc1, sc3) / 16, (sc4, sc6), (sc5, sc7) / 16
   // (odd sub-blocks hold high nibbles); NS = -1024 SC
   half2_t SC[T][4], NS[T][4];
-  uint32_t ml[T], mh[T];
+  uint32_t ml[T], mh[T], sl[T], sh8[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     uint32_t scl, sch;
     q4k_scales_packed(w[t].h.y, w[t].h.z, w[t].h.w, scl, sch, ml[t], mh[t]);
+    sl[t] = scl;
+    sh8[t] = sch;
     constexpr uint32_t nb = neg_base(0);
     const half2_t h16 = {(half_t)0.0625f, (half_t)0.0625f}, hn = {(half_t)-1024.f, (half_t)-1024.f};
     SC[t][0] = __builtin_bit_cast(half2_t, f16_codes(scl, 0x00FF00FFu, nb));
@@ -282,8 +313,23 @@ __device__ __forceinline__ void mk_unit(const Unit<12> (&w)[T], int bo, int lane
       for (int t = 0; t < T; ++t) {
         const int si = (j >> 2) * 2 + hb, sh = (j >> 1) & 1;
         const half2_t scp = {SC[t][si][sh], SC[t][si][sh]}, nsp = {NS[t][si][sh], NS[t][si][sh]};
-        const half8_t B = as_h8(mk_scaled(wq[t][0], m, base, scp, nsp), mk_scaled(wq[t][1], m, base, scp, nsp),
-                                mk_scaled(wq[t][2], m, base, scp, nsp), mk_scaled(wq[t][3], m, base, scp, nsp));
+        half8_t B;
+        if constexpr (TYPE == 13) {
+          const half_t z = (half_t)(hb ? -1280.f : -1040.f);
+          const half2_t off = {z, z};
+          uint32_t v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t q5 = i >> 1 ? w[t].qh.y : w[t].qh.x;
+            const uint32_t f = i & 1 ? (hb ? q5k_hi_odd(q5, c) : q5k_lo_odd(q5, c))
+                                     : (hb ? q5k_hi_even(q5, c) : q5k_lo_even(q5, c));
+            v[i] = mk_centred(wq[t][i], m, base, scp, off, f);
+          }
+          B = as_h8(v[0], v[1], v[2], v[3]);
+        } else {
+          B = as_h8(mk_scaled(wq[t][0], m, base, scp, nsp), mk_scaled(wq[t][1], m, base, scp, nsp),
+                    mk_scaled(wq[t][2], m, base, scp, nsp), mk_scaled(wq[t][3], m, base, scp, nsp));
+        }
 #pragma unroll
         for (int a = 0; a < MA; ++a)
           D[t][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[a], B, D[t][a], 0, 0, 0);
@@ -294,11 +340,12 @@ __device__ __forceinline__ void mk_unit(const Unit<12> (&w)[T], int bo, int lane
     }
   }
   // mins: one 16x16x16 MFMA per activation tile (K = 8 group sums x hi / lo)
-  half4_t B2[T];
+  half4_t B2[T], B3[T];  // B3, Q5_K: the scales, for the middle code's share
   float d[T], dm[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     B2[t] = mk_mins_operand((g & 1) ? mh[t] : ml[t]);
+    if constexpr (TYPE == 13) B3[t] = mk_mins_operand((g & 1) ? sh8[t] : sl[t]);
     // a slot past the wave's units (valid false) adds exactly zero
     d[t] = valid ? h2f(w[t].h.x) : 0.f;
     dm[t] = valid ? -32.f * h2f(w[t].h.x >> 16) : 0.f;
@@ -312,9 +359,17 @@ __device__ __forceinline__ void mk_unit(const Unit<12> (&w)[T], int bo, int lane
     for (int t = 0; t < T; ++t) {
       const float4_t zero = {0.f, 0.f, 0.f, 0.f};
       const float4_t D2 = __builtin_amdgcn_mfma_f32_16x16x16f16(A2, B2[t], zero, 0, 0, 0);
+      if constexpr (TYPE == 13) {
+        const float4_t D3 = __builtin_amdgcn_mfma_f32_16x16x16f16(A2, B3[t], zero, 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        acc[t][a][i] = fmaf(f[i], fmaf(d[t], D[t][a][i], dm[t] * D2[i]), acc[t][a][i]);
+        for (int i = 0; i < 4; ++i)
+          acc[t][a][i] = fmaf(f[i], fmaf(d[t], D[t][a][i], fmaf(512.f * d[t], D3[i], dm[t] * D2[i])),
+                              acc[t][a][i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[t][a][i] = fmaf(f[i], fmaf(d[t], D[t][a][i], dm[t] * D2[i]), acc[t][a][i]);
+      }
     }
     if constexpr (MA * T >= 4) __builtin_amdgcn_sched_barrier(0);  // one tile at a time
   }
@@ -475,15 +530,27 @@ __device__ __forceinline__ void mk_unit_q6k(const Unit<14> (&w)[T], int bo, int 
       for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(acc[t][a][i]));
 }
 
-// Q8_0: eight 32-element blocks per unit, each with its own scale d_b and its
-// own inverse activation scale F_b (NF = 8): one MFMA of the exact int8 codes
-// per block and activation tile, acc += (F_b d_b) D_b.
-template <int MA, int T>
-__device__ __forceinline__ void mk_unit_q8(const Q8Super (&w)[T], int bo, int lane, bool valid,
-                                           float (&acc)[T][MA][4]) {
+// The block types and IQ4_XS: eight 32-element blocks per unit, each with its own scale
+// d_b and its own inverse activation scale F_b (NF = 8): one MFMA of the exact
+// integer codes per block and activation tile, sum += (F_b d_b) D_b from zero, and one
+// addition of the unit's sum to acc.  Added to acc block by block, the range's sums have
+// four times the additions in a chain: rms error at N = 14336, K = 4096, f32 rows, Q8_0
+// 1.23e-7 then, 0.96e-7 now, Q5_0 1.26e-7 and 0.94e-7 (mb_kernel: 1.10e-7).  The empty
+// asm keeps the blocks in order; without it they are interleaved, and up to 590 registers
+// are spilled.
+template <int TYPE, int MA, int T>
+__device__ __forceinline__ void mk_unit_blocks(const typename MkUnitOf<TYPE>::type (&w)[T], int bo,
+                                               int lane, bool valid, float (&acc)[T][MA][4]) {
 #pragma clang fp contract(off)
   const int r = lane & 15, g = lane >> 4;
   const int arow = bo + r * (kMkLd * 2) + 16 * g;  // byte offset of the lane's A fragment
+  float sum[T][MA][4];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int a = 0; a < MA; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[t][a][i] = 0.f;
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
     half8_t A[MA];
@@ -495,17 +562,23 @@ __device__ __forceinline__ void mk_unit_q8(const Q8Super (&w)[T], int bo, int la
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      const half8_t B = q8_operand(w[t].b[b]);
-      const float d = valid ? h2f(w[t].b[b].d) : 0.f;  // a slot past the units adds zero
+      const half8_t B = mk_block(w[t], b, g);
+      const float d = valid ? mk_block_scale(w[t], b) : 0.f;  // a slot past the units adds zero
 #pragma unroll
       for (int a = 0; a < MA; ++a) {
         const float4_t zero = {0.f, 0.f, 0.f, 0.f};
         const float4_t D = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[a], B, zero, 0, 0, 0);
         const float f[4] = {F[a].x, F[a].y, F[a].z, F[a].w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[t][a][i] = fmaf(f[i] * d, D[i], acc[t][a][i]);
+        for (int i = 0; i < 4; ++i) sum[t][a][i] = fmaf(f[i] * d, D[i], sum[t][a][i]);
       }
     }
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int a = 0; a < MA; ++a)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(sum[t][a][i]));
     if constexpr (MA * T >= 4) __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
@@ -513,7 +586,10 @@ __device__ __forceinline__ void mk_unit_q8(const Q8Super (&w)[T], int bo, int la
 #pragma unroll
     for (int a = 0; a < MA; ++a)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(acc[t][a][i]));
+      for (int i = 0; i < 4; ++i) {
+        acc[t][a][i] += sum[t][a][i];
+        asm volatile("" : "+v"(acc[t][a][i]));
+      }
 }
 
 // Workgroup (blockIdx.x, blockIdx.y) of TS x KL waves: row tiles
@@ -686,10 +762,10 @@ __global__ __launch_bounds__(64 * TS * KL) void mk_kernel(const uint8_t *__restr
       mk_unit_iq<TYPE, MA, T>(wb[i % P], min(kl + KL * i, ulast) * UB, lane, i < cnt_u, tbl, acc);
     else if constexpr (TYPE == 14)
       mk_unit_q6k<MA, T>(wb[i % P], min(kl + KL * i, ulast) * UB, lane, i < cnt_u, acc);
-    else if constexpr (TYPE == 8)
-      mk_unit_q8<MA, T>(wb[i % P], min(kl + KL * i, ulast) * UB, lane, i < cnt_u, acc);
+    else if constexpr (mk_blocks(TYPE))
+      mk_unit_blocks<TYPE, MA, T>(wb[i % P], min(kl + KL * i, ulast) * UB, lane, i < cnt_u, acc);
     else
-      mk_unit<MA, T>(wb[i % P], min(kl + KL * i, ulast) * UB, lane, i < cnt_u, acc);
+      mk_unit<TYPE, MA, T>(wb[i % P], min(kl + KL * i, ulast) * UB, lane, i < cnt_u, acc);
     if (i + P < U)  // compile-time
 #pragma unroll
       for (int t = 0; t < T; ++t)
@@ -809,7 +885,12 @@ MkPlan mk_plan(int M, int N, int K) {
   const int ntiles = (N + 15) / 16, nu = K / 256;
   p.groups = (ntiles + p.ts * p.t - 1) / (p.ts * p.t);
   int ranges = (nu + kw_max - 1) / kw_max;
-  while (ranges < nu && (int64_t)p.groups * ranges < GGUF_MK_MIN_WGS) ++ranges;
+  // K <= 1024, up to 16 rows: one range even where few workgroups result, as the
+  // reduction's launch costs more than they do (N = 4096, K = 1024, M = 8, f32 rows:
+  // Q4_K 8.2 -> 7.1 us, Q6_K 12.0 -> 10.5, Q8_0 10.3 -> 8.7, IQ2_XXS 11.3 -> 10.0; with
+  // 32 f16 rows to convert the workgroups take longer: Q4_K 11.3 against 12.6)
+  if (!(p.sx && ranges == 1 && M <= 16))
+    while (ranges < nu && (int64_t)p.groups * ranges < GGUF_MK_MIN_WGS) ++ranges;
   p.kw = (nu + ranges - 1) / ranges;
   p.ranges = (nu + p.kw - 1) / p.kw;
   const size_t stage = ((size_t)p.kw * ub + 1023) & ~(size_t)1023;
@@ -820,7 +901,8 @@ MkPlan mk_plan(int M, int N, int K) {
   const size_t img = p.sx ? 0 : ((size_t)nu * ub + 1024 + 255) & ~(size_t)255;
   const size_t parts = p.ranges > 1 ? (size_t)p.ranges * M * ntiles * 16 * 4 : 0;
   p.part_off = (size_t)kWsPrefix + img;
-  p.bytes = img + parts > 0 ? p.part_off + parts : 0;
+  // the grid types ask for a workspace past one unit (without one they run row by row)
+  p.bytes = img + parts > 0 || (is_iq(TYPE) && nu > 1) ? p.part_off + parts : 0;
   return p;
 }
 
@@ -857,6 +939,35 @@ hipError_t launch_mk_ma(const XT *x, int64_t ldx, const uint8_t *W, int N, int K
 template <int TYPE, typename XT>
 size_t mk_work_bytes(int M, int N, int K) {
   return mk_plan<TYPE, XT>(M, N, K).bytes;
+}
+
+// Whether the batched kernel takes M rows.  Its conversion, barrier and reduction cost
+// more than mb_kernel's, so small weights of the types whose mb_kernel is good stay
+// there.  Graph replays in us, mb_kernel / mk_kernel, f32 rows unless said:
+//   Q5_K    14336 x 4096: M = 2 27.4 / 13.7, 12 32.3 / 18.2, 32 67.3 / 25.3;
+//           4096^2: 14.0 / 12.8 (M = 8); 2048^2: 9.0 / 11.4; 8192 x 2048: 13.0 / 12.4
+//           (f16 12.1 / 12.8); 14336 x 1024: 20.0 / 10.6; 4096 x 1024: 7.8 / 10.5;
+//           512 x 8192: 15.7 / 13.1
+//   IQ4_XS  8192 x 4096: 17.3 / 13.9; 4096^2 13.9 / 13.0, f16 12.0 / 12.9;
+//           14336 x 1024: 19.8 / 10.7; 512 x 8192: 15.7 / 13.6, but M = 32 18.7 / 20.9
+//   Q5_0 (Q4_0 and IQ4_NL alike)  14336 x 4096: M = 2 20.7 / 15.5, 32 54.7 / 27.9;
+//           8192 x 4096: f16 12.7 / 13.6; narrow weights, where mb_kernel has few
+//           workgroups and many slices: 1000 x 1024 13.9 / 10.7 (M = 32 15.7 / 20.3),
+//           1024 x 4096 15.4 / 13.1, 512 x 14336 34.4 / 16.2; 4096 x 2048 9.4 / 12.8
+template <int TYPE>
+bool mk_takes(int M, int N, int K) {
+  if (TYPE == 10 || TYPE == 11 || K % 256 != 0) return false;
+  const int64_t units = (int64_t)((N + 15) / 16) * (K / 256);
+  if (TYPE == 13)
+    return M > 1 && (K >= 8192 || units >= 6144 || (units >= 2048 && (M > 16 || K >= 4096)) ||
+                     (units >= 3072 && K <= 1024));
+  if (TYPE == 23)
+    return M > 1 && (units >= 6144 || (K >= 8192 && (M <= 16 || units >= 1536)) ||
+                     (units >= 3072 && K <= 1024));
+  if (TYPE == 2 || TYPE == 6 || TYPE == 20)
+    return M > 1 && ((units >= 12288 && K >= 4096) ||
+                     (N <= 1024 && K >= 1024 && (M <= 16 || K >= 4096)));
+  return true;
 }
 
 // hipErrorNotSupported (nothing launched) when the workspace is missing or

@@ -169,6 +169,56 @@ def test_batched_decode_random_blocks(pkg, ref, t, xdt):
             outs.append(y)
 
 
+@pytest.mark.parametrize("t", [13, 2, 6, 20, 23])
+@pytest.mark.parametrize("xdt", [np.float32, np.float16])
+def test_batched_decode_more_types(pkg, ref, t, xdt):
+    """As test_batched_decode_random_blocks for the other types of the batched kernel: the
+    edges of its activation tiles (8 f32 rows a tile), odd columns, several K ranges, and
+    two shapes that the rule leaves to the other kernel (a small weight, K = 4128)."""
+    lib = pkg.load_library()
+    s = torch.cuda.current_stream().cuda_stream
+    x_type = 0 if xdt == np.float32 else 1
+    shapes = [(2, 1, 8192), (8, 100, 1280), (9, 257, 8192), (16, 1000, 1280), (17, 785, 8192),
+              (24, 790, 8192), (25, 48, 12288), (32, 785, 8192), (8, 30, 512)]
+    if t in (2, 6, 20):
+        shapes.append((9, 40, 4128))
+    for i, (m, n, k) in enumerate(shapes):
+        raw = tile_model.random_blocks(t, n, k, seed=90 * t + i, specials=False)
+        x = np.random.default_rng(i).standard_normal((m, k)).astype(xdt)
+        w = pkg.repack_gguf_for_gpu(t, raw, n, k)
+        wdeq = ref.dequant_rows(t, raw, n, k)
+        xd = torch.from_numpy(x).cuda()
+        need = lib.gguf_hip_matmul_workspace(t, x_type, n, k, m)
+        x64 = x.astype(np.float64)
+        want, mag = ref.matmul_bt(x64, wdeq), ref.matmul_bt_abs(x64, wdeq)
+        for use_ws in (True, False):
+            work = torch.zeros(max(need, 16), dtype=torch.uint8, device="cuda")
+            y = torch.full((m, n), float("nan"), device="cuda")
+            assert lib.gguf_hip_matmul_ws(
+                xd.data_ptr(), x_type, k, w.ptr(), t, n, k, y.data_ptr(), n, m, DECODE,
+                work.data_ptr() if use_ws else None, need if use_ws else 0, s) == 0
+            met = ref.parity_metrics(y.cpu().numpy(), want, mag)
+            assert met["finite"] and met["elemwise"] <= DECODE_TOL, ((t, m, n, k, use_ws), met)
+
+
+@pytest.mark.parametrize("t", [8, 12, 14, 16])
+@pytest.mark.parametrize("m", [2, 16, 17])
+def test_batched_decode_short_k(pkg, ref, t, m):
+    """K <= 1024: up to 16 rows in one range, which needs no workspace (the grid types ask
+    for one all the same); past that, and past K = 1024, split over K."""
+    lib = pkg.load_library()
+    for k in (256, 1024, 1280):
+        need = lib.gguf_hip_matmul_workspace(t, 0, 40, k, m)
+        assert (need == 0) == (k == 256 or (t != 16 and k == 1024 and m <= 16))
+        raw = tile_model.random_blocks(t, 40, k, seed=t + k, specials=False)
+        w = pkg.repack_gguf_for_gpu(t, raw, 40, k)
+        x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+        y = pkg.qlinear(torch.from_numpy(x).cuda(), w).cpu().numpy()
+        x64, wdeq = x.astype(np.float64), ref.dequant_rows(t, raw, 40, k)
+        met = ref.parity_metrics(y, ref.matmul_bt(x64, wdeq), ref.matmul_bt_abs(x64, wdeq))
+        assert met["finite"] and met["elemwise"] <= DECODE_TOL, (t, m, k, met)
+
+
 def test_reference_kernel_test_shapes(pkg, ref):
     """kernel-tests.ts:910-927: M=3, N=70, K=512 per type, and N > 65535 (Q8_0, M=1, K=64)."""
     for t in (2, 6, 8, 10, 11, 12, 13, 14, 20, 23):
