@@ -17,6 +17,7 @@ cannot.
 
 from __future__ import annotations
 
+import contextlib
 import dataclasses
 from typing import Optional
 
@@ -31,7 +32,8 @@ _X_TYPES = {torch.float32: F32, torch.float16: F16}
 
 
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    # the handle itself: a torch.cuda.Stream object for it takes a microsecond more
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def _as_device_u8(data, device) -> torch.Tensor:
@@ -300,6 +302,7 @@ def _row_stride(t: torch.Tensor, rows: int, cols: int, name: str) -> int:
 _WORKSPACES: dict = {}
 _GRAPH_KEPT: list = []
 _MIN_WORKSPACE = 1 << 20
+_NO_GUARD = contextlib.nullcontext()
 
 
 def workspace_key(device_index: int, stream_handle: int, capturing: bool) -> tuple:
@@ -361,9 +364,12 @@ def dispatch_matmul_gguf(a: torch.Tensor, gg: GGUFWeight, c: torch.Tensor, M: in
     dev = gg.device
     x_type = _X_TYPES[a.dtype]
     # the split-K paths' workspace (activation image, partial sums of the K slices)
-    need = _native.check(lib.gguf_hip_matmul_workspace(gg.ggml_type, x_type, N, K, M), lib)
+    # one row of up to 16384 elements takes the one-shot kernel, which needs no workspace
+    need = 0 if M == 1 and K <= 16384 else \
+        _native.check(lib.gguf_hip_matmul_workspace(gg.ggml_type, x_type, N, K, M), lib)
     work = matmul_workspace(dev, need) if need > 0 else None
-    with torch.cuda.device(dev):
+    # the device guard costs as much as the launch; it is needed on another device only
+    with _NO_GUARD if torch.cuda.current_device() == dev.index else torch.cuda.device(dev):
         _native.check(lib.gguf_hip_matmul_ws(
             a.data_ptr() + a_off, x_type, ldx, gg.ptr(), gg.ggml_type, N, K,
             c.data_ptr() + c_off, ldy, M, variant, work.data_ptr() if work is not None else None,
