@@ -798,27 +798,52 @@ __global__ __launch_bounds__(256) void dequant_raw_kernel(const uint8_t *__restr
 }
 
 // Row gather: out[i * ldo + j] = dequant(raw row ids[i])[j].  One thread per
-// (output row, piece).  An id outside [0, n_rows) reads nothing and writes a
-// row of NaN, so a bad token id is visible in the output instead of faulting.
+// (output row, piece).  A thread's values are up to 128 neighbours, so written straight
+// out a wave's stores lie a piece apart; LDS: they go through shared memory (rows padded
+// by one word: no bank conflicts) and are stored side by side.  An id outside
+// [0, n_rows) reads nothing and writes a row of NaN, so a bad token id is visible in the
+// output instead of faulting.
+//
+// Rows of 4096 values, direct / through LDS, in us: Q4_K 1 row 4.4 / 3.7, 64 10.7 / 6.4,
+// 1900 77 / 9.4; Q6_K 1 row 6.6 / 6.8, 8 17.9 / 12.4, 1900 55 / 18.6; Q3_K (and Q2_K) 1900
+// 13.6 / 14.0; the others alike, Q8_0: 64 rows 3.4 / 3.8, 1024 9.6 /
+// 6.3, 1900 15.4 / 8.4 (the stores' pieces merge in L2 until the output outgrows it;
+// before that the detour is latency); Q5_K 1024 9.0 / 9.7, 1900 14.2 / 12.3.
 template <int TYPE>
-__global__ __launch_bounds__(256) void get_rows_kernel(const uint8_t *__restrict__ raw,
-                                                       int64_t n_rows, int64_t units_per_row,
-                                                       const int64_t *__restrict__ ids,
-                                                       int64_t n_ids, float *__restrict__ out,
-                                                       int64_t ldo) {
+constexpr bool get_rows_lds(int64_t n_ids, int64_t values) {
+  return TYPE == 12 || (TYPE == 14 && n_ids >= 8) ||
+         (TYPE != 14 && TYPE != 10 && TYPE != 11 && values >= (int64_t)(TYPE == 13 ? 3 : 2) << 21);
+}
+template <int TYPE, bool LDS>
+constexpr int get_rows_threads() { return LDS && RawPiece<TYPE>::VALUES > 64 ? 128 : 256; }
+
+template <int TYPE, bool LDS>
+__global__ __launch_bounds__((get_rows_threads<TYPE, LDS>())) void get_rows_kernel(
+    const uint8_t *__restrict__ raw, int64_t n_rows, int64_t units_per_row,
+    const int64_t *__restrict__ ids, int64_t n_ids, float *__restrict__ out, int64_t ldo) {
   using P = RawPiece<TYPE>;
-  const int64_t per_row = units_per_row * P::PER_UNIT;
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= n_ids * per_row) return;
-  const int64_t i = g / per_row, p = g % per_row;
-  const int64_t id = ids[i];
-  float *o = out + i * ldo + p * P::VALUES;
-  if (id < 0 || id >= n_rows) {
-    for (int j = 0; j < P::VALUES; ++j) o[j] = __builtin_nanf("");
-    return;
+  constexpr int V = P::VALUES, NT = get_rows_threads<TYPE, LDS>();
+  __shared__ float v[LDS ? NT * (V + 1) : 1];
+  __shared__ int64_t dst[LDS ? NT : 1];
+  const int64_t per_row = units_per_row * P::PER_UNIT, total = n_ids * per_row;
+  const int64_t g0 = (int64_t)blockIdx.x * NT, g = g0 + threadIdx.x;
+  if (g < total) {
+    const int64_t i = g / per_row, p = g - i * per_row, id = ids[i];
+    float *o = LDS ? v + threadIdx.x * (V + 1) : out + i * ldo + p * V;
+    if constexpr (LDS) dst[threadIdx.x] = i * ldo + p * V;
+    if (id < 0 || id >= n_rows) {
+      for (int j = 0; j < V; ++j) o[j] = __builtin_nanf("");
+    } else {
+      const uint8_t *unit = raw + (id * units_per_row + p / P::PER_UNIT) * Fmt<TYPE>::UB;
+      P::run(unit, (int)(p % P::PER_UNIT), o);
+    }
   }
-  const uint8_t *unit = raw + (id * units_per_row + p / P::PER_UNIT) * Fmt<TYPE>::UB;
-  P::run(unit, (int)(p % P::PER_UNIT), o);
+  if constexpr (LDS) {
+    __syncthreads();
+    const int n = (int)min((int64_t)NT, total - g0) * V;
+    for (int e = threadIdx.x; e < n; e += NT)
+      out[dst[e / V] + e % V] = v[e / V * (V + 1) + e % V];
+  }
 }
 
 template <int TYPE>
@@ -870,8 +895,16 @@ static void get_rows_type(const uint8_t *raw, int64_t n_rows, int64_t k, const i
                           int64_t n_ids, float *out, int64_t ldo, hipStream_t s) {
   const int64_t upr = k / Fmt<TYPE>::UE;
   const int64_t threads = n_ids * upr * RawPiece<TYPE>::PER_UNIT;
-  hipLaunchKernelGGL(get_rows_kernel<TYPE>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                     s, raw, n_rows, upr, ids, n_ids, out, ldo);
+  const auto launch = [&](auto lds) {
+    constexpr int NT = get_rows_threads<TYPE, decltype(lds)::value>();
+    hipLaunchKernelGGL((get_rows_kernel<TYPE, decltype(lds)::value>),
+                       dim3((unsigned)((threads + NT - 1) / NT)), dim3(NT), 0, s, raw, n_rows, upr,
+                       ids, n_ids, out, ldo);
+  };
+  if (get_rows_lds<TYPE>(n_ids, n_ids * k))
+    launch(std::true_type());
+  else
+    launch(std::false_type());
 }
 
 hipError_t launch_get_rows(const uint8_t *raw, int type, int64_t n_rows, int64_t k,

@@ -46,6 +46,21 @@ def test_get_rows_bit_exact(ref, t):
     assert np.isnan(o[1:, :k]).all() and (o[:, k:] == 0).all()
 
 
+@pytest.mark.parametrize("t", [2, 11, 12, 14, 23])
+def test_get_rows_many(ref, t):
+    """Rows that straddle workgroups, a last workgroup that is not full, strided output rows
+    of an odd stride and bad ids among good ones."""
+    n, k = 9, 768
+    raw = pkg.quantize.quantize(pkg.quantize.synthetic_weight(n, k, seed=t, std=1.0), t)
+    table = pkg.QuantEmbedding(torch.from_numpy(raw).cuda(), t, n, k)
+    ids = np.random.default_rng(t).integers(-1, n + 1, 5501)
+    out = torch.zeros(5501, k + 5, device="cuda")
+    table.gather(torch.from_numpy(ids).cuda(), out[:, :k])
+    o, good = out.cpu().numpy(), (ids >= 0) & (ids < n)
+    assert ref.same_bits(np.ascontiguousarray(o[good, :k]), ref.dequant_rows(t, raw, n, k)[ids[good]])
+    assert np.isnan(o[~good, :k]).all() and (o[:, k:] == 0).all()
+
+
 def test_loader_placement(tmp_path, ref):
     tensors = gm.make_model(seed=1, rope_freqs=True)
     extra = [("blk.0.ffn_gate_exps.weight", [256, 64, 4], 12,
