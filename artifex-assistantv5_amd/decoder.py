@@ -45,7 +45,7 @@ import numpy as np
 import torch
 
 from . import glue, quantize
-from .ggml import FUSED_TYPES, Q4_K, Q6_K, raw_row_bytes
+from .ggml import FUSED_TYPES, Q4_K, Q6_K, TILE_ROWS, raw_row_bytes
 from .linear import (GGUFWeight, LayerWeights, QuantEmbedding, concat_rows, dispatch_matmul_gguf,
                      interleave_tiles, repack_gguf_for_gpu, split_interleaved)
 
@@ -321,8 +321,10 @@ class QuantDecoder:
                                    cfg.head_dim)
             glue.add_rmsnorm(x, self._proj(att, lw.o_gg, f"L{l}-o"), lw.ffn_norm, cfg.eps, h)
             w = lw.get("gateUpI_gg")
-            if w is not None:  # tile-interleaved gate / up columns -> [gate | up] rows
-                gu = torch.cat(split_interleaved(self._proj(h, w, f"L{l}-gateUp")), dim=1)
+            if w is not None:  # tile-interleaved gate / up columns -> [gate | up] rows, one copy
+                gu = torch.empty(M, 2, cfg.ffn // TILE_ROWS, TILE_ROWS, device=self.device)
+                gu.copy_(self._proj(h, w, f"L{l}-gateUp").view(M, -1, 2, TILE_ROWS).transpose(1, 2))
+                gu = gu.view(M, 2 * cfg.ffn)
             else:
                 gu = self._proj_slot(h, lw, "gateUp", f"L{l}-gateUp")
             glue.swiglu(gu, a)
