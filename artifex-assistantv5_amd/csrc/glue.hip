@@ -8,7 +8,6 @@
 // All kernels are f32, one row (or one KV head) per workgroup; they are small
 // and latency-bound, so the goal is one launch per op with coalesced 16-byte
 // accesses, not occupancy.
-#include <climits>
 #include <mutex>
 
 #include "common.hpp"
@@ -370,47 +369,40 @@ __global__ __launch_bounds__(kGlueThreads) void attention_kernel(
 // lies outside 0..max_seq-1 writes nothing.
 //
 // attention_prefill_kernel: causal GQA attention of each row over slots
-// 0..pos[m] (attention.wgsl:60-234 with new_seq_len = M), flash-style, in f32
-// grade on the f16 matrix cores: an f32 operand, scaled by a power of two,
-// enters as f16 hi + lo (22 significant bits) and a product is hi hi + hi lo +
-// lo hi, accumulated in f32.
-// - A wave takes 32 rows of one query head; a workgroup takes four consecutive
-//   (32-row block, head of the group) pairs of one KV head, so that groups of
-//   any size fill it.  Blocks are launched last rows first (the longest causal
-//   ranges), KV head fastest: with 8 KV heads each XCD keeps one head's K and V
-//   in its L2.
-// - Keys come in tiles of KT slots.  Wave w converts the w-th quarter (group) of
-//   the tile, each group with a power of two of their own (K and V apart), so
-//   the conversion needs no cross-wave maximum.  K rows and transposed V rows,
-//   hi and lo, are stored in LDS, rows padded by 16 bytes: every fragment read
-//   is one base register and an immediate, free of bank conflicts.
-// - Two barriers per tile: V's loads are in flight under S = K Q, the next K's
-//   under O += V P, so a wave holds one operand's 8 float4 at a time.
-// - S^T = K . Q^T (keys x rows): in the 32x32x16 accumulator, lane l holds keys
-//   8 (r / 4) + 4 (l / 32) + r % 4 of row l % 32.  V^T is stored with the middle
-//   two of each four 4-key blocks exchanged, so that those registers, converted
-//   to f16, are the B operand of O^T += V^T . P^T: the probabilities never
-//   leave their lane.
-// - log2 e is folded into the score factor; the running maximum is rounded up
-//   to an integer, so a rescale is by an exact power of two, and it is skipped
-//   while no row's maximum moved.
-// What bounds it: the vector work of the conversion and the softmax beside the
-// matrix cores' three products (per 64 keys and 32 rows about 3900 cycles of VALU
-// issue against 3072 of MFMA), and few workgroups.  Against the v_mfma f32 kernel
-// it replaces (16 rows per wave, f32 K / V tiles): 1500 rows over 548 cached, 32 / 8
-// heads of 128, 584 -> 158 us with the append; 500 rows over 1500, 8 / 2 heads of
-// 64 / 128 / 256, 119 -> 85, 218 -> 134, 417 -> 273; 8 rows over 700, 83 -> 54.  The
-// error against float64 fell from 7.2e-7 to 4.6e-7 there (fewer, longer f32
-// accumulation steps), and is no larger at any of 37 shapes tried.
+// 0..pos[m] (attention.wgsl:60-234 with new_seq_len = M), flash-style on the
+// f32 matrix cores.
+// - A workgroup takes 16 rows and one KV head.  Wave w takes query heads
+//   w, w + 4, ... of the group, one per pass over the keys.
+// - Keys come in tiles of KT slots: K rows [KT][HD + 4] and V transposed
+//   [HD][KT + 4] in LDS.  The next tile's loads are in flight while the
+//   current tile is used.
+// - Per 16 keys, v_mfma_f32_16x16x4f32 computes S^T = K . Q^T (keys x rows).
+//   Its accumulator layout (lane l: keys 4(l/16) + r of row l%16) is exactly
+//   the B-operand layout of O^T += V^T . P^T when k-step r takes keys
+//   4(l/16) + r.  So the probabilities never leave their registers.
+// - Every lane holds one row's running max, running sum and output column,
+//   so the online-softmax rescale is lane-local.
+// - The head_dim reduction of S^T runs over elements 16a + 4(l/16) + b, a
+//   bijection onto 0..HD-1, so each lane's K and Q operands are float4 reads.
+// - Every operand is f32: a key that a row does not see adds an exact zero to it,
+//   whatever the key holds (up to overflow).  f16 hi + lo operands with exponents shared
+//   by the keys of a group are three times as fast, but there a later row's large key
+//   takes the bits of earlier rows' keys and values.
+// - Workgroups are launched last rows first (the longest causal ranges), KV head
+//   fastest: 1500 rows over 548 cached, 32 / 8 heads of 128, 595 us in row order, 462 so;
+//   1900 rows, 12 / 4 heads of 128, 336 and 221; 500 rows over 1500 or fewer rows alike.
+// What bounds it: the f32 matrix cores (a sixteenth of the f16 rate) with two waves per
+// SIMD to fill them (LDS).
 // A row whose position lies outside 0..max_seq-1, or past M, attends to
 // nothing and is not written.
-constexpr int kPfRows = 32;   // rows (positions) per wave
-constexpr int kPfWaves = 4;   // (row block, head) pairs per workgroup
-// key slots per tile, a quarter of them per wave
-template <int HD>
-constexpr int pf_keys() { return HD <= 128 ? 64 : 32; }
+constexpr int kPfRows = 16;  // rows (positions) per workgroup
 
-typedef float float16_t __attribute__((ext_vector_type(16)));
+template <int HD>
+struct PfShape {
+  static constexpr int KT = HD <= 128 ? 64 : 32;          // key slots per tile
+  static constexpr int KLD = HD + 4, VLD = KT + 4;         // LDS row strides (floats)
+  static constexpr int NF = KT * HD / 4 / kGlueThreads;    // float4 of K (and of V) per thread
+};
 
 template <int HD>
 __global__ __launch_bounds__(kGlueThreads) void rope_append_kernel(
@@ -436,391 +428,175 @@ __global__ __launch_bounds__(kGlueThreads) void rope_append_kernel(
   }
 }
 
-__device__ __forceinline__ float16_t mfma_h32(half8_t a, half8_t b, float16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-// The power of two 2^e that brings a largest magnitude m to [2^13, 2^14), e
-// clamped to +-126.
-__device__ __forceinline__ int pf_exp(float m) {
-  const int e = 140 - (int)((__float_as_uint(m) >> 23) & 255u);
-  return max(-126, min(126, e));
-}
-__device__ __forceinline__ float pf_pow2(int e) {  // 2^e, |e| <= 126
-  return __uint_as_float((uint32_t)(e + 127) << 23);
-}
-
-// f16 hi + lo parts of eight f32 values times sc
-__device__ __forceinline__ void pf_split(const float *x, float sc, half8_t &hi, half8_t &lo) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    float v = x[i] * sc;
-    asm("" : "+v"(v));  // one product for both parts (else it is folded into each conversion)
-    const half_t h = (half_t)v;
-    hi[i] = h;
-    lo[i] = (half_t)(v - (float)h);
-  }
-}
-
-// Largest finite magnitude of a wave's n values (an infinity must not take the
-// scale from the finite values of its group; NaN never wins).
-template <int N>
-__device__ __forceinline__ float pf_wave_absmax(const float (&x)[N]) {
-  float m = 0.f;
-#pragma unroll
-  for (int i = 0; i < N; ++i) m = fmaxf(m, fabsf(x[i]));
-  m = max_xor32(max_xor16(max_lanes16(m)));
-  if (__builtin_amdgcn_readfirstlane(__float_as_uint(m)) == 0x7f800000u) {
-    m = 0.f;
-#pragma unroll
-    for (int i = 0; i < N; ++i) m = fmaxf(m, fabsf(x[i]) < INFINITY ? fabsf(x[i]) : 0.f);
-    m = max_xor32(max_xor16(max_lanes16(m)));
-  }
-  return m;
-}
-
-// A wave's 32 query rows of one head, roped and split: qh / ql[s] = the f16 hi /
-// lo parts of elements 16 s + 8 (lane / 32) + 0..7 of row lane % 32, times 2^eq
-// (the row's own exponent).  Returns log2 e / sqrt(HD) * 2^-eq.  A row is read by
-// HD / 8 lanes side by side (a lane per row would read 32 lines per load) and
-// turned through the wave's part of LDS, ROWS rows at a time.  `my`: the lane's row's position, or -1 (zeros).
-template <int HD>
-struct PfQuery {
-  static constexpr int LPR = HD / 8, RPG = 64 / LPR;   // lanes per row, rows per load
-  static constexpr int ROWS = HD <= 128 ? 32 : 16;     // rows per pass
-  static constexpr int RB = 2 * HD + 16, BYTES = 2 * ROWS * RB;
-};
-
-template <int HD>
-__device__ __forceinline__ float pf_query(const float *__restrict__ qrows, int64_t ldq,
-                                          const float *__restrict__ cs,
-                                          const float *__restrict__ sn, int my, unsigned char *buf,
-                                          half8_t (&qh)[HD / 16], half8_t (&ql)[HD / 16]) {
-  using Q = PfQuery<HD>;
-  constexpr int half = HD / 2, NG = Q::ROWS / Q::RPG;
-  const int lane = threadIdx.x & 63, col = lane & 31, hf = lane >> 5;
-  const int i = 4 * (lane % Q::LPR);
-  int eq = 0;
-  if (Q::ROWS < kPfRows) {  // a pass without rows is left out
-#pragma unroll
-    for (int k = 0; k < HD / 16; ++k)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) qh[k][e] = ql[k][e] = (half_t)0.f;
-  }
-#pragma unroll
-  for (int r0 = 0; r0 < kPfRows; r0 += Q::ROWS) {
-    if (Q::ROWS < kPfRows && !__any(my >= 0 && col / Q::ROWS * Q::ROWS == r0)) continue;
-    float4 a[NG], b[NG], c[NG], s[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      const int row = r0 + g * Q::RPG + lane / Q::LPR, p = __shfl(my, row);
-      a[g] = b[g] = c[g] = s[g] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (p >= 0) {
-        const float *q = qrows + row * ldq + i;
-        a[g] = *(const float4 *)q;
-        b[g] = *(const float4 *)(q + half);
-        c[g] = *(const float4 *)(cs + (int64_t)p * half + i);
-        s[g] = *(const float4 *)(sn + (int64_t)p * half + i);
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      const int row = g * Q::RPG + lane / Q::LPR;
-      float x[8] = {a[g].x * c[g].x - b[g].x * s[g].x, a[g].y * c[g].y - b[g].y * s[g].y,
-                    a[g].z * c[g].z - b[g].z * s[g].z, a[g].w * c[g].w - b[g].w * s[g].w,
-                    b[g].x * c[g].x + a[g].x * s[g].x, b[g].y * c[g].y + a[g].y * s[g].y,
-                    b[g].z * c[g].z + a[g].z * s[g].z, b[g].w * c[g].w + a[g].w * s[g].w};
-      float mx = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(x[e]));
-      mx = fmaxf(mx, dpp<kDppXor1>(mx));
-      mx = fmaxf(mx, dpp<kDppXor2>(mx));
-      mx = fmaxf(mx, dpp<kDppHalfMirror>(mx));
-      if (Q::LPR >= 16) mx = fmaxf(mx, dpp<kDppMirror>(mx));
-      if (Q::LPR >= 32) mx = max_xor16(mx);
-      const int e2 = pf_exp(mx);
-      half8_t h, l;
-      pf_split(x, pf_pow2(e2), h, l);
-      unsigned char *at = buf + row * Q::RB + 2 * i;
-      *(half4_t *)at = half4_t{h[0], h[1], h[2], h[3]};
-      *(half4_t *)(at + HD) = half4_t{h[4], h[5], h[6], h[7]};
-      at += Q::ROWS * Q::RB;
-      *(half4_t *)at = half4_t{l[0], l[1], l[2], l[3]};
-      *(half4_t *)(at + HD) = half4_t{l[4], l[5], l[6], l[7]};
-      if (lane % Q::LPR == 0) *(int *)(buf + row * Q::RB + 2 * HD) = e2;  // in the row's pad
-    }
-    // the wave's own LDS writes are visible to it in program order
-    if (Q::ROWS == kPfRows || col / Q::ROWS * Q::ROWS == r0) {
-      const unsigned char *at = buf + (col - r0) * Q::RB;
-      eq = *(const int *)(at + 2 * HD);
-#pragma unroll
-      for (int k = 0; k < HD / 16; ++k) {
-        qh[k] = *(const half8_t *)(at + 32 * k + 16 * hf);
-        ql[k] = *(const half8_t *)(at + Q::ROWS * Q::RB + 32 * k + 16 * hf);
-      }
-    }
-  }
-  return 1.44269504088896340736f / sqrtf((float)HD) * pf_pow2(-eq);
+__device__ __forceinline__ float4_t mfma_f32(float a, float b, float4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
 template <int HD>
-__global__ __launch_bounds__(64 * kPfWaves, HD <= 128 ? 2 : 1) void attention_prefill_kernel(
+__global__ __launch_bounds__(kGlueThreads) void attention_prefill_kernel(
     const float *__restrict__ qkv, int64_t ldq, const int64_t *__restrict__ pos, int64_t M,
     const float *__restrict__ cs, const float *__restrict__ sn, const float *__restrict__ kc,
     const float *__restrict__ vc, float *__restrict__ out, int64_t ldo, int nh, int nkv,
     int max_seq) {
-  constexpr int KS = HD / 16;                 // k steps of S
-  constexpr int DT = HD / 32;                 // 32-wide output tiles
-  constexpr int KT = pf_keys<HD>(), GK = KT / kPfWaves;  // keys per tile, per wave's group
-  constexpr int JT = KT / 32;                 // 32-key score tiles
-  constexpr int KRB = 2 * HD + 16, VRB = 2 * KT + 16;  // bytes of a K row and of a V^T row in LDS
-  constexpr int KI = GK * HD / 8 / 64;        // 8-element chunks of K per lane
-  constexpr int NB = GK / 4;                  // 4-key blocks of a group
-  constexpr int VI = NB * HD / 4 / 64;        // 4 x 4 blocks of V per lane
-  constexpr int CPR = HD / 8;                 // chunks per K row
-  __shared__ __align__(16) unsigned char lds[2 * KT * KRB + 2 * HD * VRB];
-  unsigned char *const kh = lds, *const kl = kh + KT * KRB;
-  unsigned char *const vh = kl + KT * KRB, *const vl = vh + HD * VRB;
-  __shared__ int kex[kPfWaves], vex[kPfWaves], kends[kPfWaves];
+  using Sh = PfShape<HD>;
+  constexpr int KT = Sh::KT, KLD = Sh::KLD, VLD = Sh::VLD, NF = Sh::NF, half = HD / 2;
+  constexpr int QA = HD / 16;  // float4 of q per lane, and 16-element output tiles
+  constexpr int NT = KT / 16;  // 16-key tiles per key tile
+  __shared__ __align__(16) float ks[KT * KLD];
+  __shared__ __align__(16) float vt[HD * VLD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int col = lane & 31, hf = lane >> 5;  // MFMA column (row of the block), k half
-  const int grp = nh / nkv, kvh = blockIdx.x;
-  const int64_t unit = (int64_t)(gridDim.y - 1 - blockIdx.y) * kPfWaves + wave;
-  const int64_t rb = unit / grp;
-  const int jh = (int)(unit - rb * grp);
-  const int64_t m = rb * kPfRows + col;
+  const int col = lane & 15, g4 = lane >> 4;  // MFMA column (row of the block), k group
+  // the workgroups in launch order: KV head fastest, the last rows first
+  const int64_t b = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  const int grp = nh / nkv, kvh = (int)(b % nkv);
+  const int64_t m = ((int64_t)gridDim.x - 1 - b / nkv) * kPfRows + col;
   int my = -1;  // the row's position; -1: attends to nothing, not written
   if (m < M) {
     const int64_t p = pos[m];
     if (p >= 0 && p < max_seq) my = (int)p;
   }
-  // slots 0 .. wend - 1 hold every key of the wave's rows, slots up to wlo are
-  // seen by all of them
-  int wend = my + 1, wlo = my >= 0 ? my : INT_MAX;
+  // slots 0 .. kend - 1 hold every key of the block's rows (same in every wave)
+  int kend = my + 1;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    wend = max(wend, __shfl_xor(wend, o));
-    wlo = min(wlo, __shfl_xor(wlo, o));
-  }
-  if (lane == 0) kends[wave] = wend;
-  __syncthreads();
-  int kend = 0;
-#pragma unroll
-  for (int w = 0; w < kPfWaves; ++w) kend = max(kend, kends[w]);
-  kend = __builtin_amdgcn_readfirstlane(kend);
-  wend = __builtin_amdgcn_readfirstlane(wend);
-  wlo = __builtin_amdgcn_readfirstlane(wlo);
-  if (kend == 0) return;  // the whole workgroup: no row attends to anything
+  for (int o = 32; o > 0; o >>= 1) kend = max(kend, __shfl_xor(kend, o));
   const int ntile = (kend + KT - 1) / KT;
   const float *kbase = kc + (int64_t)kvh * max_seq * HD;
   const float *vbase = vc + (int64_t)kvh * max_seq * HD;
-  // wave w's share of a tile: keys GK w + ..; a slot past the last key re-reads
-  // that key (its score is masked, its probability 0)
-  float kr[8 * KI];
-  auto load_k = [&](int t0) {
+  const float scale = 1.0f / sqrtf((float)HD);
+
+  // float4 f = i * 256 + tid of a tile: 64-float4 block f / 64 = (16-slot block,
+  // 4-chunk block); within it slot f % 16, chunk (f / 16) % 4.  A wave's LDS
+  // stores (K rows, V transposed) are then free of bank conflicts.
+  float4 kr[NF], vr[NF];
+  auto load_tile = [&](int t0) {
 #pragma unroll
-    for (int i = 0; i < KI; ++i) {
-      const int f = i * 64 + lane, t = GK * wave + f / CPR, c = f % CPR;
-      const float *src = kbase + (int64_t)min(t0 + t, kend - 1) * HD + 8 * c;
-      *(float4 *)(kr + 8 * i) = *(const float4 *)src;
-      *(float4 *)(kr + 8 * i + 4) = *(const float4 *)(src + 4);
+    for (int i = 0; i < NF; ++i) {
+      const int f = i * kGlueThreads + tid, blk = f >> 6;
+      const int t = (blk / (HD / 16)) * 16 + (f & 15), c = (blk % (HD / 16)) * 4 + ((f >> 4) & 3);
+      const int row = t0 + t;  // < kend <= max_seq when read
+      kr[i] = row < kend ? *(const float4 *)(kbase + (int64_t)row * HD + 4 * c)
+                         : make_float4(0.f, 0.f, 0.f, 0.f);
+      vr[i] = row < kend ? *(const float4 *)(vbase + (int64_t)row * HD + 4 * c)
+                         : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   };
-  auto store_k = [&]() {
-    const int e = pf_exp(pf_wave_absmax(kr));
-    if (lane == 0) kex[wave] = e;
-    const float sc = pf_pow2(e);
+  auto store_tile = [&]() {
 #pragma unroll
-    for (int i = 0; i < KI; ++i) {
-      const int f = i * 64 + lane, t = GK * wave + f / CPR, c = f % CPR;
-      half8_t h, l;
-      pf_split(kr + 8 * i, sc, h, l);
-      const int at = t * KRB + 16 * c;
-      *(half8_t *)(kh + at) = h;
-      *(half8_t *)(kl + at) = l;
+    for (int i = 0; i < NF; ++i) {
+      const int f = i * kGlueThreads + tid, blk = f >> 6;
+      const int t = (blk / (HD / 16)) * 16 + (f & 15), c = (blk % (HD / 16)) * 4 + ((f >> 4) & 3);
+      *(float4 *)(ks + t * KLD + 4 * c) = kr[i];
+      vt[(4 * c + 0) * VLD + t] = vr[i].x;
+      vt[(4 * c + 1) * VLD + t] = vr[i].y;
+      vt[(4 * c + 2) * VLD + t] = vr[i].z;
+      vt[(4 * c + 3) * VLD + t] = vr[i].w;
     }
   };
-  // V: 4 keys x 4 elements per block, transposed in registers
-  auto load_v = [&](int t0) {
+
+  for (int hp = 0; hp * 4 < grp; ++hp) {
+    const int jh = hp * 4 + wave;  // query head within the group
+    const bool act = jh < grp;     // wave-uniform
+    const int64_t qcol = (int64_t)(kvh * grp + jh) * HD + 4 * g4;
+    // the row's query, roped and scaled: q[a] = elements 16a + 4 g4 + 0..3
+    float4 q[QA];
 #pragma unroll
-    for (int i = 0; i < VI; ++i) {
-      const int b = NB * wave + lane % NB, c = lane / NB + 64 / NB * i;
+    for (int a = 0; a < QA; ++a) q[a] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (act && my >= 0) {
+      const float *qin = qkv + m * ldq + qcol;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        *(float4 *)(kr + 16 * i + 4 * e) =
-            *(const float4 *)(vbase + (int64_t)min(t0 + 4 * b + e, kend - 1) * HD + 4 * c);
+      for (int a = 0; a < QA; ++a) q[a] = *(const float4 *)(qin + 16 * a);
+      const float *crow = cs + (int64_t)my * half + 4 * g4, *srow = sn + (int64_t)my * half + 4 * g4;
+#pragma unroll
+      for (int a = 0; a < QA / 2; ++a) {
+        const float4 c = *(const float4 *)(crow + 16 * a), s = *(const float4 *)(srow + 16 * a);
+        const float4 x = q[a], y = q[a + QA / 2];
+        q[a] = make_float4((x.x * c.x - y.x * s.x) * scale, (x.y * c.y - y.y * s.y) * scale,
+                           (x.z * c.z - y.z * s.z) * scale, (x.w * c.w - y.w * s.w) * scale);
+        q[a + QA / 2] =
+            make_float4((y.x * c.x + x.x * s.x) * scale, (y.y * c.y + x.y * s.y) * scale,
+                        (y.z * c.z + x.z * s.z) * scale, (y.w * c.w + x.w * s.w) * scale);
+      }
     }
-  };
-  auto store_v = [&]() {
-    const int e = pf_exp(pf_wave_absmax(kr));
-    if (lane == 0) vex[wave] = e;
-    const float sc = pf_pow2(e);
+    float4_t o[QA];
 #pragma unroll
-    for (int i = 0; i < VI; ++i) {
-      const int b = NB * wave + lane % NB, c = lane / NB + 64 / NB * i;
+    for (int a = 0; a < QA; ++a) o[a] = float4_t{0.f, 0.f, 0.f, 0.f};
+    float mrun = -INFINITY, lrun = 0.f;
+
+    if (ntile > 0) load_tile(0);
+    for (int it = 0; it < ntile; ++it) {
+      __syncthreads();  // every wave is done with the previous tile
+      store_tile();
+      __syncthreads();
+      if (it + 1 < ntile) load_tile((it + 1) * KT);
+      if (!act) continue;
+      // S^T for the tile's keys: s[j][r] = score of key it*KT + 16j + 4 g4 + r
+      float4_t s[NT];
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        half4_t h, l;
+      for (int j = 0; j < NT; ++j) {
+        s[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+        const float *kp = ks + (16 * j + col) * KLD + 4 * g4;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          float v = kr[16 * i + 4 * k + d] * sc;
-          asm("" : "+v"(v));
-          h[k] = (half_t)v;
-          l[k] = (half_t)(v - (float)h[k]);
+        for (int a = 0; a < QA; ++a) {
+          const float4 kf = *(const float4 *)(kp + 16 * a);
+          s[j] = mfma_f32(kf.x, q[a].x, s[j]);
+          s[j] = mfma_f32(kf.y, q[a].y, s[j]);
+          s[j] = mfma_f32(kf.z, q[a].z, s[j]);
+          s[j] = mfma_f32(kf.w, q[a].w, s[j]);
         }
-        const int at = (4 * c + d) * VRB + 32 * (b >> 2) + 16 * (b & 1) + 8 * ((b >> 1) & 1);
-        *(half4_t *)(vh + at) = h;
-        *(half4_t *)(vl + at) = l;
       }
-    }
-  };
-
-  load_k(0);  // in flight under the query's loads
-  half8_t qh[KS], ql[KS];
-  const float qf = pf_query<HD>(qkv + rb * kPfRows * ldq + (int64_t)(kvh * grp + jh) * HD, ldq, cs,
-                                sn, my, kh + wave * PfQuery<HD>::BYTES, qh, ql);
-  static_assert(kPfWaves * PfQuery<HD>::BYTES <= 2 * KT * KRB + 2 * HD * VRB, "fits in the tile");
-  __syncthreads();  // the queries' staging is read: the tile may be written
-  float16_t o[DT];
-#pragma unroll
-  for (int a = 0; a < DT; ++a)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[a][r] = 0.f;
-  float mrun = -INFINITY, lrun = 0.f;
-  int evrun = 126, evmin = 126;  // exponent of the accumulator's V, smallest so far
-
-  store_k();
-  for (int it = 0; it < ntile; ++it) {
-    const int t0 = it * KT;
-    const bool act = t0 < wend;  // wave-uniform
-    __syncthreads();             // K of this tile stored, V of the previous one read
-    load_v(t0);
-    float16_t s[JT];
-    float alpha = 1.f;
-    if (act) {
-      const unsigned char *kp = kh + col * KRB + 16 * hf, *kq = kl + col * KRB + 16 * hf;
-      half8_t ah = *(const half8_t *)kp, al = *(const half8_t *)kq;
-#pragma unroll
-      for (int n = 0; n < JT * KS; ++n) {  // the next fragments are read ahead of the MFMAs
-        const int j = n / KS, k = n % KS, n1 = n + 1 < JT * KS ? n + 1 : n;
-        const int at = 32 * (n1 / KS) * KRB + 32 * (n1 % KS);
-        const half8_t bh = *(const half8_t *)(kp + at), bl = *(const half8_t *)(kq + at);
-        if (k == 0)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) s[j][r] = 0.f;
-        s[j] = mfma_h32(al, qh[k], s[j]);
-        s[j] = mfma_h32(ah, ql[k], s[j]);
-        s[j] = mfma_h32(ah, qh[k], s[j]);
-        ah = bh;
-        al = bl;
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x8, 3, 0);
-      }
-      // score factors of the tile's key groups, kept normal (a masked -inf
-      // times 0 would be NaN)
-      float f[kPfWaves];
-#pragma unroll
-      for (int g = 0; g < kPfWaves; ++g)
-        f[g] = fminf(fmaxf(qf * pf_pow2(-kex[g]), 0x1p-126f), 0x1p126f);
-      if (t0 + KT - 1 > wlo) {  // some row does not see the whole tile
-#pragma unroll
-        for (int j = 0; j < JT; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (t0 + 32 * j + 8 * (r >> 2) + 4 * hf + (r & 3) > my) s[j][r] = -INFINITY;
-      }
+      // causal mask, the block's max over the row (4 lanes share a row)
+      const int tb = it * KT + 4 * g4;
       float bm = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < JT; ++j)
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; r += 4)
-          bm = fmaxf(bm, fmaxf(fmaxf(s[j][r], s[j][r + 1]), fmaxf(s[j][r + 2], s[j][r + 3])) *
-                             f[(32 * j + 2 * r) / GK]);
-      bm = max_xor32(bm);
-      const float mnew = fmaxf(mrun, ceilf(bm));
-      const float mu = mnew == -INFINITY ? 0.f : mnew;
-      alpha = __builtin_amdgcn_exp2f(mrun - mu);  // an exact power of two, 0 at the start
+        for (int r = 0; r < 4; ++r) {
+          const float v = tb + 16 * j + r <= my ? s[j][r] : -INFINITY;
+          s[j][r] = v;
+          bm = fmaxf(bm, v);
+        }
+      bm = fmaxf(bm, __shfl_xor(bm, 16));
+      bm = fmaxf(bm, __shfl_xor(bm, 32));
+      const float mnew = fmaxf(mrun, bm);
+      const float alpha = mnew == -INFINITY ? 1.f : expf(mrun - mnew);
       mrun = mnew;
       float ls = 0.f;
 #pragma unroll
-      for (int j = 0; j < JT; ++j)
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float e = __builtin_amdgcn_exp2f(fmaf(s[j][r], f[(32 * j + 8 * (r >> 2)) / GK], -mu));
+        for (int r = 0; r < 4; ++r) {
+          const float e = s[j][r] == -INFINITY ? 0.f : expf(s[j][r] - mnew);
           s[j][r] = e;
           ls += e;
         }
-      lrun = fmaf(lrun, alpha, ls);
-    }
-    store_v();
-    __syncthreads();  // V stored, every wave is done with K
-    if (it + 1 < ntile) load_k(t0 + KT);
-    if (act) {
-      // the accumulator's scale follows V's: down at once when a group holds
-      // larger values, up once all are 2^8 smaller (never above 2^60 of the
-      // largest seen, so that it cannot overflow)
-      int emin = vex[0];
+      lrun = lrun * alpha + ls;
 #pragma unroll
-      for (int g = 1; g < kPfWaves; ++g) emin = min(emin, vex[g]);
-      emin = __builtin_amdgcn_readfirstlane(emin);
-      evmin = min(evmin, emin);
-      const int en = emin < evrun || emin > evrun + 8 ? min(emin, evmin + 60) : evrun;
-      const float rs = ldexpf(alpha, en - evrun);  // exact; 0 at the wave's first tile
-      evrun = en;
-      if (__any(rs != 1.f)) {
+      for (int a = 0; a < QA; ++a) o[a] *= alpha;
+      // O^T[d][row] += sum over the tile's keys of V[key][d] P[row][key]
 #pragma unroll
-        for (int a = 0; a < DT; ++a)
+      for (int j = 0; j < NT; ++j) {
+        const float *vp = vt + col * VLD + 16 * j + 4 * g4;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) o[a][r] *= rs;
-      }
-      float pf[kPfWaves];
-#pragma unroll
-      for (int g = 0; g < kPfWaves; ++g)
-        pf[g] = ldexpf(0x1p15f, evrun - __builtin_amdgcn_readfirstlane(vex[g]));
-      const unsigned char *vp = vh + col * VRB + 16 * hf, *vq = vl + col * VRB + 16 * hf;
-      half8_t bh = *(const half8_t *)vp, bl = *(const half8_t *)vq;
-      half8_t ph[2], pl[2];
-      // probabilities times 2^(15 + evrun - vex) <= 2^15: each group's V has its own exponent
-      auto split_p = [&](int g) {
-        float p[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          p[i] = s[g >> 1][8 * (g & 1) + i] * pf[(16 * g + 8 * (i >> 2)) / GK];
-        pf_split(p, 1.f, ph[g & 1], pl[g & 1]);
-      };
-      split_p(0);
-#pragma unroll
-      for (int n = 0; n < KT / 16 * DT; ++n) {
-        const int g = n / DT, a = n % DT, n1 = n + 1 < KT / 16 * DT ? n + 1 : n;
-        const int at = 32 * (n1 % DT) * VRB + 32 * (n1 / DT);
-        const half8_t ch = *(const half8_t *)(vp + at), cl = *(const half8_t *)(vq + at);
-        if (a == 0 && g + 1 < KT / 16) split_p(g + 1);
-        o[a] = mfma_h32(bl, ph[g & 1], o[a]);
-        o[a] = mfma_h32(bh, pl[g & 1], o[a]);
-        o[a] = mfma_h32(bh, ph[g & 1], o[a]);
-        bh = ch;
-        bl = cl;
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+        for (int a = 0; a < QA; ++a) {
+          const float4 vf = *(const float4 *)(vp + 16 * a * VLD);
+          o[a] = mfma_f32(vf.x, s[j][0], o[a]);
+          o[a] = mfma_f32(vf.y, s[j][1], o[a]);
+          o[a] = mfma_f32(vf.z, s[j][2], o[a]);
+          o[a] = mfma_f32(vf.w, s[j][3], o[a]);
         }
       }
     }
-    if (it + 1 < ntile) store_k();
-  }
-  float l = lrun + __shfl_xor(lrun, 32);
-  if (my >= 0) {
-    const float inv = 1.0f / l;
-    float *orow = out + m * ldo + (int64_t)(kvh * grp + jh) * HD + 4 * hf;
+    if (!act) continue;
+    float l = lrun + __shfl_xor(lrun, 16);
+    l += __shfl_xor(l, 32);
+    if (my >= 0) {
+      const float inv = 1.0f / l;
+      float *orow = out + m * ldo + qcol;
 #pragma unroll
-    for (int a = 0; a < DT; ++a)
-#pragma unroll
-      for (int r = 0; r < 16; r += 4)
-        *(float4 *)(orow + 32 * a + 2 * r) = make_float4(
-            ldexpf(o[a][r] * inv, -15 - evrun), ldexpf(o[a][r + 1] * inv, -15 - evrun),
-            ldexpf(o[a][r + 2] * inv, -15 - evrun), ldexpf(o[a][r + 3] * inv, -15 - evrun));
+      for (int a = 0; a < QA; ++a)
+        *(float4 *)(orow + 16 * a) = make_float4(o[a][0] * inv, o[a][1] * inv, o[a][2] * inv,
+                                                 o[a][3] * inv);
+    }
   }
 }
 
@@ -1021,9 +797,8 @@ static hipError_t launch_prefill_hd(const float *qkv, int64_t ldq, const int64_t
                      ldq, pos, cs, sn, kc, vc, nh, nkv, max_seq);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int64_t units = (m + kPfRows - 1) / kPfRows * (nh / nkv);
-  const dim3 grid((unsigned)nkv, (unsigned)((units + kPfWaves - 1) / kPfWaves));
-  hipLaunchKernelGGL(attention_prefill_kernel<HD>, grid, dim3(64 * kPfWaves), 0, s, qkv, ldq, pos,
+  const dim3 grid((unsigned)((m + kPfRows - 1) / kPfRows), (unsigned)nkv);
+  hipLaunchKernelGGL(attention_prefill_kernel<HD>, grid, dim3(kGlueThreads), 0, s, qkv, ldq, pos,
                      m, cs, sn, kc, vc, out, ldo, nh, nkv, max_seq);
   return hipGetLastError();
 }

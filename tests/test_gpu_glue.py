@@ -219,10 +219,10 @@ def test_attention_prefill_edges(lib, nh, nkv, hd, max_seq, m, pos0, scale):
     and values of each 4 slots carry a power of two of their own in 2^-12 .. 2^12
     and the queries 2^-8, and a key no row sees is infinite.
 
-    Bound, with u = 2^-24: an operand's hi + lo parts hold it to 2 u and the dropped
-    lo lo product is below 4 u of its term, so a score is within 16 u sum |q k| and
-    the f32 sums of it and of hd (RoPE included) products add less than that again;
-    a probability moves by its score's error, and the sum of p v by its own.  In
+    Bound, with u = 2^-24: a score is an f32 chain of hd products (RoPE: two roundings
+    more each), whose rounding errors are below u of sum |q k| a step and add up as a
+    random walk, to 16 u for hd = 256; a probability moves by its score's error, and the
+    sum of p v, a chain over the keys, by as much again.  Four times that, in
     ratio to sum p |v|: 64 u (1 + max sum |q k| / sqrt(hd))."""
     g = torch.Generator(device="cuda").manual_seed(hd + m)
     row, orow, grp, half = (nh + 2 * nkv) * hd, nh * hd, nh // nkv, hd // 2
@@ -257,3 +257,46 @@ def test_attention_prefill_edges(lib, nh, nkv, hd, max_seq, m, pos0, scale):
         lim = 64 * 2.0 ** -24 * (1 + mag)[:, None] * (p @ v.abs())
         assert torch.isfinite(out[:, h * hd:(h + 1) * hd]).all()
         assert (err <= lim).all(), (h, (err / lim).max().item())
+
+
+@pytest.mark.parametrize("nh,nkv,hd,m,pos0", [(4, 1, 128, 100, 37), (2, 2, 64, 70, 0),
+                                              (4, 2, 256, 50, 20), (16, 2, 128, 40, 300)])
+@pytest.mark.parametrize("ek,ev", [(20, -30), (-40, 24), (60, 60)])
+def test_attention_prefill_later_keys(lib, nh, nkv, hd, m, pos0, ek, ev):
+    """What later rows hold does not reach earlier rows: with the keys of the rows from r0
+    on times 2^ek (their queries 2^-ek) and the values 2^ev, the rows before r0 keep their
+    bits.  The later rows, whose values differ by 2^ev within a tile, are held to the bound
+    of test_attention_prefill_edges."""
+    g = torch.Generator(device="cuda").manual_seed(hd + m)
+    row, orow, grp, half = (nh + 2 * nkv) * hd, nh * hd, nh // nkv, hd // 2
+    r0, max_seq = m // 2 + 3, pos0 + m
+    plain = torch.randn(m, row, device="cuda", generator=g)
+    later = plain.clone()
+    later[r0:, :orow] *= 2.0 ** -ek
+    later[r0:, orow:orow + nkv * hd] *= 2.0 ** ek
+    later[r0:, orow + nkv * hd:] *= 2.0 ** ev
+    kc0 = torch.randn(nkv, max_seq, hd, device="cuda", generator=g)
+    vc0 = torch.randn(nkv, max_seq, hd, device="cuda", generator=g)
+    inv, cos, sin = _rope_inv(hd, max_seq)
+    pos = torch.arange(pos0, max_seq, device="cuda")
+    outs = []
+    for qkv in (plain, later):
+        kc, vc = kc0.clone(), vc0.clone()
+        out = torch.full((m, orow), float("nan"), device="cuda")
+        _ok(lib, lib.gguf_hip_attention_prefill(
+            qkv.data_ptr(), row, pos.data_ptr(), m, cos.data_ptr(), sin.data_ptr(), kc.data_ptr(),
+            vc.data_ptr(), out.data_ptr(), orow, nh, nkv, hd, max_seq, _s()))
+        outs.append(out)
+    assert torch.equal(outs[0][:r0], outs[1][:r0])
+    c, s = cos[pos].double()[:, None], sin[pos].double()[:, None]
+    q = later[:, :orow].double().view(m, nh, hd)
+    a, b = q[..., :half], q[..., half:]
+    q = torch.cat([a * c - b * s, b * c + a * s], dim=-1)[r0:]
+    masked = torch.arange(max_seq, device="cuda")[None] > pos[r0:, None]
+    for h in range(nh):
+        k, v = kc[h // grp].double(), vc[h // grp].double()
+        sc = (q[:, h] @ k.T / math.sqrt(hd)).masked_fill(masked, float("-inf"))
+        mag = (q[:, h].abs() @ k.abs().T / math.sqrt(hd)).masked_fill(masked, 0).amax(1)
+        p = torch.softmax(sc, dim=1)
+        err = (outs[1][r0:, h * hd:(h + 1) * hd].double() - p @ v).abs()
+        assert (err <= 64 * 2.0 ** -24 * (1 + mag)[:, None] * (p @ v.abs())).all()
