@@ -417,12 +417,19 @@ namespace gguf {
 //   M = max_s m_s,  w_s = exp(m_s - M),  L = sum_s w_s l_s,
 //   out = (sum_s w_s o_s) * (1 / L).
 constexpr int kAttnSplit = 64;
-// Up to kMergeChunk splits (of max_seq) the output projection merges the records
-// in its prologue; longer caches take attn_merge_kernel and the plain projection.
-constexpr int kMergeChunk = 8;
+// Caches of up to kMergeMax splits: the output projection merges the records in its
+// prologue, kMergeChunk at a time.  Longer ones: attn_merge_kernel (glue.hip) writes the
+// merged output behind the records, and the prologue reads that.  The launch costs about
+// 3 us a layer at any position; the prologue nothing up to 8 records and then 0.4 us each,
+// every workgroup reading them all.  A short range in a cache of ordinary size must not pay
+// for long ones: 4 layers of d 4096, 32 / 8 heads of 128, a step at position 10 / 300 /
+// 700 / 1000 / 2000 with the launch 224 / 227 / 235 / 237 / 242 us, with the prologue 211 /
+// 219 / 235 / 243 / 271 (one record at a time 210 / 219 / 241 / 253 / 299).  At 6000 the
+// prologue, one at a time, takes 495, the launch 282.
+constexpr int kMergeChunk = 8, kMergeMax = 32;
 constexpr int attn_record_stride(int hd) { return hd + 4; }
 struct AttnRecords {
-  const float *work;     // the records
+  const float *work;     // the records, then (S > kMergeMax) the merged output [nh][hd]
   const int64_t *pos;    // device position p; the range holds slots 0..p
   int nh, nkv, hd;       // query heads, KV heads, head dim
   int max_seq;
@@ -473,8 +480,6 @@ hipError_t launch_rmsnorm(float *x, const float *r, const float *w, float eps, f
 hipError_t launch_swiglu(const float *gu, float *out, int64_t rows, int64_t ffn, hipStream_t s);
 int64_t attention_work_bytes(int nh, int nkv, int hd, int64_t max_seq);
 int64_t attention_noalloc_bytes(int nh, int nkv, int hd, int64_t max_seq);
-// Merges the records into the workspace; *merged = the output [nh * hd].
-hipError_t launch_attn_merge(const AttnRecords &ar, const float **merged, hipStream_t s);
 hipError_t launch_attention_decode(const float *qkv, const int64_t *pos, const float *cs,
                                    const float *sn, float *kc, float *vc, float *out, float *work,
                                    int nh, int nkv, int hd, int64_t max_seq, hipStream_t s);

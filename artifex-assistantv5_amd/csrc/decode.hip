@@ -31,17 +31,9 @@ hipError_t launch_decode_fused(const float *x, const uint8_t *tiles, int type, i
 }
 
 // The attention output projection with the record merge as its prologue
-// (decode_m1_kernel, PRO 3): K = nh * hd.  A cache of more than kMergeChunk
-// splits is merged by a launch of its own.
+// (decode_m1_kernel, PRO 3): K = nh * hd.
 hipError_t launch_decode_attn_merge(const AttnRecords &ar, const uint8_t *tiles, int type,
                                     int64_t n, float *y, int epi, hipStream_t s) {
-  if ((ar.max_seq + kAttnSplit - 1) / kAttnSplit > kMergeChunk) {
-    const float *x = nullptr;
-    const hipError_t e = launch_attn_merge(ar, &x, s);
-    if (e != hipSuccess) return e;
-    return launch_decode_fused(x, tiles, type, n, (int64_t)ar.nh * ar.hd, y, 0, nullptr, 0.f, epi,
-                               s);
-  }
   switch (type) {
     case 2: return decode_merge_q4_0(ar, tiles, (int)n, y, epi, s);
     case 6: return decode_merge_q5_0(ar, tiles, (int)n, y, epi, s);

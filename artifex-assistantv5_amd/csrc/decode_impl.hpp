@@ -1414,6 +1414,9 @@ int64_t mb_work_floats(int M, int N, int K) {
 //            own): each thread's item is a 16-element slice of one query
 //            head, and its records (at most kMergeChunk splits) are
 //            requested with the activations, ahead of the weights;
+//   PRO = 4  the same for caches of more splits: the records past the first
+//            kMergeChunk are requested that many at a time, and of a cache of more
+//            than kMergeMax splits the merged output is read (attn_merge_kernel);
 // and the epilogue `epi`:
 //   0  y = result;
 //   1  y += result (the residual add after the output and down projections);
@@ -1484,37 +1487,56 @@ __global__ __launch_bounds__(512) void decode_m1_kernel(const XT *__restrict__ x
 #pragma unroll
   for (int i = 0; i < XI; ++i) {
     const int q = (int)threadIdx.x + nthr * i;
-    if constexpr (PRO != 3) load_item<XT>(x, 0, K, 0, per_row, per_row, q, xv[i]);
+    if constexpr (PRO < 3) load_item<XT>(x, 0, K, 0, per_row, per_row, q, xv[i]);
     if constexpr (PRO == 1) load_item<float>(pw, 0, K, 0, per_row, per_row, q, pv[i]);
     if constexpr (PRO == 2) load_item<float>((const float *)x + K, 0, K, 0, per_row, per_row, q, pv[i]);
   }
-  // PRO 3: the item's 16-element slice of the attention records of its query
+  // PRO 3, 4: the item's 16-element slice of the attention records of its query
   // head (the slots past the range are not loaded and get weight zero)
-  constexpr int RC = PRO == 3 ? kMergeChunk : 1;
-  float4 ro[PRO == 3 ? XI : 1][RC][4];
-  float2 rml[PRO == 3 ? XI : 1][RC];
+  constexpr int RC = PRO >= 3 ? kMergeChunk : 1, RM = PRO == 4 ? kMergeMax / 4 : 1;
+  float4 ro[PRO >= 3 ? XI : 1][RC][4];
+  float2 rml[PRO >= 3 ? XI : 1][RC];
+  float rm[PRO == 4 ? XI : 1][RM];  // past RC records: m of every (hd / 16)th, by lane
+  const float *rec0[PRO >= 3 ? XI : 1];  // the item's slice in split 0's record
   int mn = 0;              // records to merge: ceil((p + 1) / kAttnSplit), 0 for a bad p
-  if constexpr (PRO == 3) {
-    const int64_t p = ar.pos[0];
-    mn = (p >= 0 && p < ar.max_seq) ? (int)(p / kAttnSplit) + 1 : 0;
+  int64_t rstride = 0;     // floats from one split's record to the next
+  bool premerged = false;  // uniform
+  if constexpr (PRO >= 3) {
     const int grp = ar.nh / ar.nkv, S = (ar.max_seq + kAttnSplit - 1) / kAttnSplit;
     const int rs = attn_record_stride(ar.hd);
-    const int64_t rstride = (int64_t)grp * rs;  // floats from one split's record to the next
-    const int last = mn > 0 ? mn - 1 : 0;
+    rstride = (int64_t)grp * rs;
+    premerged = PRO == 4 && S > kMergeMax;
+    const int64_t p = ar.pos[0];
+    if (premerged) {  // requested without waiting for the position
 #pragma unroll
-    for (int i = 0; i < XI; ++i) {
-      const int q = min((int)threadIdx.x + nthr * i, per_row - 1);
-      const int k0 = kItem * q, h = k0 / ar.hd, i0 = k0 - h * ar.hd;
-      const int gk = h / grp, jh = h - gk * grp;
-      const float *rec = ar.work + ((int64_t)gk * S * grp + jh) * rs;
+      for (int i = 0; i < XI; ++i)
+        load_item<float>(ar.work + (int64_t)ar.nkv * S * rstride, 0, K, 0, per_row, per_row,
+                         (int)threadIdx.x + nthr * i, xv[i]);
+    }
+    mn = (p >= 0 && p < ar.max_seq) ? (int)(p / kAttnSplit) + 1 : 0;
+    if (!premerged) {
+      const int last = mn > 0 ? mn - 1 : 0;
 #pragma unroll
-      for (int c = 0; c < RC; ++c) {
-        if (c > last) break;  // uniform: the loads of splits past the range are not issued
-        const int64_t off = (int64_t)c * rstride;
-        const float4 *o4 = (const float4 *)(rec + i0 + off);
+      for (int i = 0; i < XI; ++i) {
+        const int q = min((int)threadIdx.x + nthr * i, per_row - 1);
+        const int k0 = kItem * q, h = k0 / ar.hd, i0 = k0 - h * ar.hd;
+        const int gk = h / grp, jh = h - gk * grp;
+        rec0[i] = ar.work + ((int64_t)gk * S * grp + jh) * rs + i0;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) ro[i][c][v] = o4[v];
-        rml[i][c] = *(const float2 *)(rec + ar.hd + off);
+        for (int c = 0; c < RC; ++c) {
+          if (c > last) break;  // uniform: the loads of splits past the range are not issued
+          const int64_t off = (int64_t)c * rstride;
+          const float4 *o4 = (const float4 *)(rec0[i] + off);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) ro[i][c][v] = o4[v];
+          rml[i][c] = *(const float2 *)(rec0[i] - i0 + ar.hd + off);
+        }
+        if (PRO == 4 && last >= RC) {  // past the range: the last one's
+          const int gl = ar.hd / kItem;  // lanes of a head: 4, 8 or 16
+#pragma unroll
+          for (int k = 0; k < RM; ++k)
+            rm[i][k] = rec0[i][ar.hd - i0 + min(((int)threadIdx.x & (gl - 1)) + gl * k, last) * rstride];
+        }
       }
     }
   }
@@ -1566,32 +1588,69 @@ __global__ __launch_bounds__(512) void decode_m1_kernel(const XT *__restrict__ x
         xv[i][e] = pv[i][e] * (gt / (1.0f + expf(-gt)));
       }
   }
-  if constexpr (PRO == 3) {  // merge in split order (attention_kernel's merge, same arithmetic)
+  if constexpr (PRO >= 3) {  // merge in split order (attention_kernel's merge, same arithmetic)
+    if (premerged) {
+      if (mn == 0)  // no cache slot
 #pragma unroll
-    for (int i = 0; i < XI; ++i) {
-      float M = -INFINITY;
+        for (int i = 0; i < XI; ++i)
 #pragma unroll
-      for (int c = 0; c < RC; ++c)
-        if (c < mn) M = fmaxf(M, rml[i][c].x);
-      float L = 0.f, a[kItem];
+          for (int e = 0; e < kItem; ++e) xv[i][e] = __builtin_nanf("");
+    } else {
 #pragma unroll
-      for (int e = 0; e < kItem; ++e) a[e] = 0.f;
+      for (int i = 0; i < XI; ++i) {
+        const int i0 = kItem * min((int)threadIdx.x + nthr * i, per_row - 1) % ar.hd;
+        const float *ml0 = rec0[i] - i0 + ar.hd;
+        float M = -INFINITY;
 #pragma unroll
-      for (int c = 0; c < RC; ++c) {
-        if (c >= mn) break;  // uniform; the slots past the range were never loaded
-        const float w = expf(rml[i][c].x - M);
-        L = fmaf(w, rml[i][c].y, L);
+        for (int c = 0; c < RC; ++c)
+          if (c < mn) M = fmaxf(M, rml[i][c].x);
+        if (PRO == 4 && mn > RC) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          a[4 * v] = fmaf(w, ro[i][c][v].x, a[4 * v]);
-          a[4 * v + 1] = fmaf(w, ro[i][c][v].y, a[4 * v + 1]);
-          a[4 * v + 2] = fmaf(w, ro[i][c][v].z, a[4 * v + 2]);
-          a[4 * v + 3] = fmaf(w, ro[i][c][v].w, a[4 * v + 3]);
+          for (int k = 0; k < RM; ++k) M = fmaxf(M, rm[i][k]);
+          M = fmaxf(M, dpp<kDppXor1>(M));
+          M = fmaxf(M, dpp<kDppXor2>(M));
+          if (ar.hd >= 128) M = fmaxf(M, dpp<kDppHalfMirror>(M));
+          if (ar.hd >= 256) M = fmaxf(M, dpp<kDppMirror>(M));
         }
-      }
-      const float inv = 1.0f / L;  // no records (bad position): 0 * inf = NaN
+        float L = 0.f, a[kItem];
 #pragma unroll
-      for (int e = 0; e < kItem; ++e) xv[i][e] = a[e] * inv;
+        for (int e = 0; e < kItem; ++e) a[e] = 0.f;
+        const auto load = [&](int c, int s) {
+          const float4 *o4 = (const float4 *)(rec0[i] + s * rstride);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) ro[i][c][v] = o4[v];
+          rml[i][c] = *(const float2 *)(ml0 + s * rstride);
+        };
+        for (int s0 = 0;;) {
+#pragma unroll
+          for (int c = 0; c < RC; ++c) {
+            if (s0 + c >= mn) break;  // uniform; the slots past the range were never loaded
+            const float w = expf(rml[i][c].x - M);
+            L = fmaf(w, rml[i][c].y, L);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              a[4 * v] = fmaf(w, ro[i][c][v].x, a[4 * v]);
+              a[4 * v + 1] = fmaf(w, ro[i][c][v].y, a[4 * v + 1]);
+              a[4 * v + 2] = fmaf(w, ro[i][c][v].z, a[4 * v + 2]);
+              a[4 * v + 3] = fmaf(w, ro[i][c][v].w, a[4 * v + 3]);
+            }
+          }
+          if (PRO == 3 || (s0 += RC) >= mn) break;
+          if (s0 + RC / 2 < mn) {  // the next records, straight-line (past the range: the last)
+#pragma unroll
+            for (int c = 0; c < RC; ++c) load(c, min(s0 + c, mn - 1));
+          } else {  // few: every workgroup reads them, so no more than there are
+#pragma unroll
+            for (int c = 0; c < RC / 2; ++c) {
+              if (s0 + c >= mn) break;  // uniform
+              load(c, s0 + c);
+            }
+          }
+        }
+        const float inv = 1.0f / L;  // no records (bad position): 0 * inf = NaN
+#pragma unroll
+        for (int e = 0; e < kItem; ++e) xv[i][e] = a[e] * inv;
+      }
     }
   }
 #pragma unroll
@@ -1816,7 +1875,7 @@ hipError_t launch_m1(const XT *x, const uint8_t *W, int N, int K, float *y, cons
     else if (per <= 16) GGUF_M1(16, 1);
     else if (per <= 32) GGUF_M1(32, 1);
     else GGUF_M1(64, 1);
-  } else if constexpr (PRO != 3) {
+  } else if constexpr (PRO < 3) {
     if (per <= 4) GGUF_M1(4, 2);
     else if (per <= 8) GGUF_M1(8, 2);
     else if (per <= 16) GGUF_M1(16, 2);
@@ -1875,7 +1934,9 @@ hipError_t launch_m(const XT *x, int64_t ldx, const uint8_t *W, int N, int K, fl
   }                                                                                              \
   hipError_t decode_merge_##NAME(const AttnRecords &ar, const uint8_t *tiles, int n, float *y,   \
                                  int epi, hipStream_t s) {                                       \
-    return launch_m1<T, float, 3>(nullptr, tiles, n, ar.nh * ar.hd, y, nullptr, 0.f, epi, ar, s); \
+    return ar.max_seq <= kMergeChunk * kAttnSplit                                                \
+               ? launch_m1<T, float, 3>(nullptr, tiles, n, ar.nh * ar.hd, y, nullptr, 0.f, epi, ar, s) \
+               : launch_m1<T, float, 4>(nullptr, tiles, n, ar.nh * ar.hd, y, nullptr, 0.f, epi, ar, s); \
   }
 
 // The grid-codebook IQ types: the one-shot kernel for M = 1 (K <= 16384), the
@@ -1926,7 +1987,9 @@ hipError_t launch_iq(const XT *x, int64_t ldx, const uint8_t *W, int N, int K, f
   }                                                                                              \
   hipError_t decode_merge_##NAME(const AttnRecords &ar, const uint8_t *tiles, int n, float *y,   \
                                  int epi, hipStream_t s) {                                       \
-    return launch_m1<T, float, 3>(nullptr, tiles, n, ar.nh * ar.hd, y, nullptr, 0.f, epi, ar, s); \
+    return ar.max_seq <= kMergeChunk * kAttnSplit                                                \
+               ? launch_m1<T, float, 3>(nullptr, tiles, n, ar.nh * ar.hd, y, nullptr, 0.f, epi, ar, s) \
+               : launch_m1<T, float, 4>(nullptr, tiles, n, ar.nh * ar.hd, y, nullptr, 0.f, epi, ar, s); \
   }
 
 }  // namespace gguf

@@ -677,10 +677,9 @@ hipError_t launch_swiglu(const float *gu, float *out, int64_t rows, int64_t ffn,
 // known (records past the range are read and not used): one memory round trip
 // for caches of up to 64 splits, one more per further 64.  A position outside the
 // cache gives NaN.
-// Merged in the output projection's prologue instead, every record past the chunk
-// costs each of its workgroups a memory round trip: 94 splits, 4096 x 4096 Q4_K,
-// 66.9 us with the projection against 7.4 + 5.6 for this kernel and the plain
-// projection.  The records through LDS, 1024 threads per head: 9.3 - 10.7 us.
+// For caches of more than kMergeMax splits: 94 splits, 4096 x 4096 Q4_K, one record at a
+// time in the projection's prologue 66.9 us, this kernel and the projection 7.4 + 5.6.
+// The records through LDS, 1024 threads per head: 9.3 - 10.7 us.
 constexpr int kMergeRecs = 64;
 
 template <int HD>
@@ -725,40 +724,37 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float *__restrict_
   out[(int64_t)h * HD + c] = o * (1.0f / L);
 }
 
-// Workspace: the records [nkv][S][grp][hd + 4] floats, the merged output of
-// launch_attn_merge [nh][hd] (more than kMergeChunk splits), then nkv counters.
+// Workspace: the records [nkv][S][grp][hd + 4] floats, the merged output [nh][hd] (more
+// than kMergeMax splits), then nkv counters.
 static int64_t attention_record_bytes(int nh, int nkv, int hd, int64_t max_seq) {
   const int64_t S = (max_seq + kSplit - 1) / kSplit;
   return (int64_t)sizeof(float) * nkv * S * (nh / nkv) * attn_record_stride(hd);
 }
-
-// the counters, and all that a call with an output needs
 static int64_t attention_counter_bytes(int nkv) { return ((int64_t)nkv * 4 + 15) / 16 * 16; }
 
+// what a call with an output needs
 int64_t attention_noalloc_bytes(int nh, int nkv, int hd, int64_t max_seq) {
   return attention_record_bytes(nh, nkv, hd, max_seq) + attention_counter_bytes(nkv);
 }
 
 int64_t attention_work_bytes(int nh, int nkv, int hd, int64_t max_seq) {
-  const bool merge = (max_seq + kSplit - 1) / kSplit > kMergeChunk;  // launch_attn_merge's output
+  const bool merge = (max_seq + kSplit - 1) / kSplit > kMergeMax;
   return attention_noalloc_bytes(nh, nkv, hd, max_seq) + (merge ? (int64_t)sizeof(float) * nh * hd : 0);
 }
 
-hipError_t launch_attn_merge(const AttnRecords &ar, const float **merged, hipStream_t s) {
-  float *out = (float *)((char *)ar.work +
-                         attention_record_bytes(ar.nh, ar.nkv, ar.hd, ar.max_seq));
-  const int S = (ar.max_seq + kSplit - 1) / kSplit, grp = ar.nh / ar.nkv;
-  const dim3 grid((unsigned)ar.nh, (unsigned)(ar.hd / 64)), block(64);
-  if (ar.hd == 64)
-    hipLaunchKernelGGL(attn_merge_kernel<64>, grid, block, 0, s, ar.work, ar.pos, out, grp, S,
-                       ar.max_seq);
-  else if (ar.hd == 128)
-    hipLaunchKernelGGL(attn_merge_kernel<128>, grid, block, 0, s, ar.work, ar.pos, out, grp, S,
-                       ar.max_seq);
-  else
-    hipLaunchKernelGGL(attn_merge_kernel<256>, grid, block, 0, s, ar.work, ar.pos, out, grp, S,
-                       ar.max_seq);
-  *merged = out;
+template <int HD>
+static hipError_t launch_attention_hd(const float *qkv, const int64_t *pos, const float *cs,
+                                      const float *sn, float *kc, float *vc, float *out,
+                                      float *work, unsigned *counters, int nh, int nkv,
+                                      int64_t max_seq, hipStream_t s) {
+  const int S = (int)((max_seq + kSplit - 1) / kSplit);
+  hipLaunchKernelGGL(attention_kernel<HD>, dim3((unsigned)nkv, (unsigned)S), dim3(kGlueThreads), 0,
+                     s, qkv, pos, cs, sn, kc, vc, out, work, counters, nh, nkv, (int)max_seq);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || out || S <= kMergeMax) return e;
+  float *merged = (float *)((char *)work + attention_record_bytes(nh, nkv, HD, max_seq));
+  hipLaunchKernelGGL(attn_merge_kernel<HD>, dim3((unsigned)nh, HD / 64), dim3(64), 0, s, work, pos,
+                     merged, nh / nkv, S, (int)max_seq);
   return hipGetLastError();
 }
 
@@ -766,18 +762,11 @@ static hipError_t launch_attention(const float *qkv, const int64_t *pos, const f
                                    const float *sn, float *kc, float *vc, float *out, float *work,
                                    unsigned *counters, int nh, int nkv, int hd, int64_t max_seq,
                                    hipStream_t s) {
-  const int S = (int)((max_seq + kSplit - 1) / kSplit);
-  const dim3 grid((unsigned)nkv, (unsigned)S), block(kGlueThreads);
   if (hd == 64)
-    hipLaunchKernelGGL(attention_kernel<64>, grid, block, 0, s, qkv, pos, cs, sn, kc, vc, out,
-                       work, counters, nh, nkv, (int)max_seq);
-  else if (hd == 128)
-    hipLaunchKernelGGL(attention_kernel<128>, grid, block, 0, s, qkv, pos, cs, sn, kc, vc, out,
-                       work, counters, nh, nkv, (int)max_seq);
-  else
-    hipLaunchKernelGGL(attention_kernel<256>, grid, block, 0, s, qkv, pos, cs, sn, kc, vc, out,
-                       work, counters, nh, nkv, (int)max_seq);
-  return hipGetLastError();
+    return launch_attention_hd<64>(qkv, pos, cs, sn, kc, vc, out, work, counters, nh, nkv, max_seq, s);
+  if (hd == 128)
+    return launch_attention_hd<128>(qkv, pos, cs, sn, kc, vc, out, work, counters, nh, nkv, max_seq, s);
+  return launch_attention_hd<256>(qkv, pos, cs, sn, kc, vc, out, work, counters, nh, nkv, max_seq, s);
 }
 
 hipError_t launch_attention_decode(const float *qkv, const int64_t *pos, const float *cs,

@@ -22,8 +22,8 @@ separate dispatches).  A decode step runs the glue as libgguf_hip kernels
 that consume them, the residual adds as accumulate epilogues of the output
 and down projections, RoPE + KV append + GQA attention as one launch whose
 records the output projection merges, argmax) over preallocated buffers: five
-launches per layer (six with caches of more than 512 slots, whose records are
-merged first).  Prefill (many positions at once) runs the glue as
+launches per layer (six with caches of more than 2048 slots, whose records the
+attention call merges).  Prefill (many positions at once) runs the glue as
 libgguf_hip kernels too: RMSNorm rows, each residual add fused with the
 RMSNorm after it, RoPE + KV append + causal GQA attention of all rows
 (``glue.attention_prefill``, the reference's attention.wgsl with

@@ -265,8 +265,9 @@ int gguf_hip_swiglu(const float *gate_up, float *out, int64_t rows, int64_t ffn,
  * zero-filled once before its first use, and every call leaves the counters
  * at zero again.  Calls that share a workspace must not overlap.  The
  * position is read on the device, so the call can be captured in a graph.
- * out == NULL: only the records are written (no merge, counters untouched),
- * for gguf_hip_matmul_attn_merge to merge inside the output projection. */
+ * out == NULL: only the records are written (counters untouched), for
+ * gguf_hip_matmul_attn_merge to merge inside the output projection; with more
+ * than 2048 slots a second launch merges them behind the records in `work`. */
 int gguf_hip_attention_decode(const float *qkv, const int64_t *pos, const float *cos_table,
                               const float *sin_table, float *k_cache, float *v_cache, float *out,
                               int n_heads, int n_kv_heads, int head_dim, int64_t max_seq,
@@ -320,9 +321,7 @@ int gguf_hip_attention_prefill(const float *qkv, int64_t ldqkv, const int64_t *p
  * the reference's attention-output and o-projection dispatches
  * (forward-pass.ts:2925-3297) by one.  The shapes are those of the attention
  * call; K = n_heads * head_dim <= 8192.  A position outside 0..max_seq - 1
- * gives NaN outputs.  One launch up to 512 cache slots; longer caches take two,
- * the first of which merges the records into the workspace (so work is written,
- * the records are not). */
+ * gives NaN outputs.  One launch; `work` is only read. */
 int gguf_hip_matmul_attn_merge(const void *work, const int64_t *pos, int n_heads, int n_kv_heads,
                                int head_dim, int64_t max_seq, const void *tiles, int ggml_type,
                                int64_t n, float *y, int epilogue, void *stream);

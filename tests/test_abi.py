@@ -281,7 +281,8 @@ def test_attn_merge_errors(lib, native):
     assert f(wk, pos, 3, 1, 64, 512, w, 12, 64, y, 1, None) == native.ERR_SHAPE     # K=192 % 256
     assert f(wk, pos, 32, 8, 128, 512, w, 12, 64, y, 2, None) == native.ERR_SHAPE   # SwiGLU epi
     assert "epilogue 2" in native.last_error(lib)
-    assert f(wk, pos, 64, 8, 256, 512, w, 12, 64, y, 1, None) == native.ERR_SHAPE   # K=16384
+    for max_seq in (512, 4096):
+        assert f(wk, pos, 64, 8, 256, max_seq, w, 12, 64, y, 1, None) == native.ERR_SHAPE   # K=16384
     assert "no merge kernel" in native.last_error(lib)
     assert f(None, pos, 32, 8, 128, 512, w, 12, 64, y, 1, None) == native.ERR_NULL
     assert f(wk, None, 32, 8, 128, 512, w, 12, 64, y, 1, None) == native.ERR_NULL

@@ -152,7 +152,7 @@ def _attention_inputs(nh, nkv, hd, max_seq, p):
 
 
 # positions: one split, a full split, two splits, the register chunk of eight
-# splits exactly, and caches of more splits (a merge launch)
+# splits exactly, and ranges of more splits
 @pytest.mark.parametrize("t,nh,nkv,hd,max_seq,p", [
     (12, 32, 8, 128, 1200, 0), (12, 32, 8, 128, 1200, 63), (12, 32, 8, 128, 1200, 64),
     (12, 32, 8, 128, 1200, 300), (12, 32, 8, 128, 1200, 511), (12, 32, 8, 128, 1200, 1199),
@@ -176,13 +176,38 @@ def test_attention_merge_projection_n4096_small_blocks(mods, t, p):
     _merge_case(mods, t, 32, 8, 128, 600, p, 4096)
 
 
-# caches past the prologue's eight splits are merged by a launch of their own, 64
-# records at a time: nine splits, and ranges of 63, 64, 65, 128 and 130 records
+# nine splits in the prologue, and caches past its 32 splits, which the attention call
+# merges 64 records at a time: 63, 64, 65, 128 and 130 records
 @pytest.mark.parametrize("nh,nkv,hd,max_seq,p", [
     (8, 2, 128, 513, 512), (8, 2, 128, 576, 3), (4, 4, 64, 8300, 4031), (2, 1, 256, 8300, 4095),
     (2, 1, 128, 8300, 4096), (4, 2, 64, 8192, 8191), (2, 1, 256, 8300, 8299)])
 def test_attention_merge_launch(mods, nh, nkv, hd, max_seq, p):
     _merge_case(mods, 12 if nh * hd % 256 == 0 else 8, nh, nkv, hd, max_seq, p, 256)
+
+
+# the largest cache that the prologue merges, at its chunks' edges, the smallest that the
+# attention call merges, and short ranges in long caches
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 128), (4, 4, 64), (2, 1, 256)])
+@pytest.mark.parametrize("max_seq,p", [(2048, 2047), (2048, 1000), (2048, 1023), (2048, 1024),
+                                       (2048, 100), (2049, 2047), (2049, 2048), (8300, 0),
+                                       (8300, 600)])
+def test_attention_merge_long_caches(mods, nh, nkv, hd, max_seq, p):
+    """The projection only reads the workspace, and a position outside the cache gives NaN."""
+    pkg, glue = mods
+    t = 12 if nh * hd % 256 == 0 else 8
+    _merge_case(mods, t, nh, nkv, hd, max_seq, p, 256)
+    work = glue.attention_workspace(nh, nkv, hd, max_seq, "cuda")
+    qkv, kc, vc, cos, sin = _attention_inputs(nh, nkv, hd, max_seq, p)
+    pos = torch.tensor([p], device="cuda")
+    w, y = _weight(pkg, t, 256, nh * hd, seed=p), torch.empty(256, device="cuda")
+    glue.attention_decode(qkv, pos, cos, sin, kc, vc, None, nh, nkv, hd, work)
+    before = work.clone()
+    glue.matmul_attn_merge(work, pos, w, y, nh, nkv, hd, max_seq)
+    assert torch.equal(work.view(torch.int32), before.view(torch.int32))
+    pos.fill_(max_seq)
+    glue.attention_decode(qkv, pos, cos, sin, kc, vc, None, nh, nkv, hd, work)
+    glue.matmul_attn_merge(work, pos, w, y, nh, nkv, hd, max_seq)
+    assert torch.isnan(y).all()
 
 
 def _merge_case(mods, t, nh, nkv, hd, max_seq, p, n):
