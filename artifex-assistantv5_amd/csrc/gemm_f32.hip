@@ -23,11 +23,11 @@
 //   per K half, one barrier per half unit; K half 1 runs half a unit behind.
 // - v_mfma_f32_16x16x32_f16: a fragment read from LDS feeds NT tiles, a weight
 //   operand 4 row tiles and both parts.  The operand is the exact f16 integer
-//   sc (q - Z) (Q6_K: see its operand); the codes come straight from memory.
+//   sc (q - Z) (Q6_K: the sum of two); the codes come straight from memory.
 // Measured against the 32-row passes, whole call: Q4_K 128 x 28672 x 4096
-// 146 -> 83 us, Q6_K 387 x 4096 x 14336 313 -> 205, Q5_K 200 x 14336 x 4096 427 -> 132,
-// Q6_K 500 x 14336 x 4096 464 -> 240, Q4_K 40 x 4096 x 4096 30 -> 24; the error against
-// float64 fell (Q4_K 3.0e-7 -> 1.9e-7, Q6_K 1.25e-7 -> 1.14e-7).  What bounds it: the
+// 146 -> 77 us, Q6_K 387 x 4096 x 14336 313 -> 188, Q5_K 200 x 14336 x 4096 415 -> 120,
+// Q6_K 500 x 14336 x 4096 424 -> 232, Q4_K 40 x 4096 x 4096 26 -> 22; the error against
+// float64 fell (Q4_K 3.0e-7 -> 1.9e-7, Q6_K 1.25e-7 -> 1.09e-7).  What bounds it: the
 // vector work of the operands (35 of the 78 us of the first, by leaving it out) and
 // the MFMAs beside it (28 us at their full rate) hardly overlap on two waves per SIMD.
 #include "decode_impl.hpp"
@@ -81,7 +81,7 @@ __device__ __forceinline__ uint32_t pk_fma(half2_t a, half2_t b, half2_t c) {
 __device__ __forceinline__ half2_t dup(half_t v) { return half2_t{v, v}; }
 
 // A wave's weights: NT row tiles of 16 weight rows (output columns).  PARTS = 1:
-// one exact f16 integer for both parts of x; 3: see Q6_K.
+// one exact f16 integer; 2: the sum of two (Q6_K).
 // ORDER: the k order of the activations (decode_mk.hpp).
 //   load<HF>(u)   request half HF's codes of unit u; header(u) its header
 //   begin(act)    the header as the operands use it; the unit adds zero unless act
@@ -181,14 +181,13 @@ struct FW<12> : FWK<12> {};
 template <>
 struct FW<13> : FWK<13> {};
 
-// Q6_K: W = sc (q - 32), |W| <= 4096, has up to 13 bits.  Three products: x_hi Wc with
-// Wc = W rounded to a multiple of 16 (8 bits: with x_hi's 11 the sums hardly round),
-// x_hi (W - Wc), and x_lo Wr with Wr = W rounded to f16 (x_lo's own rounding is as
-// large as what that leaves out).  Step n of a half is a window of 32 elements, the
+// Q6_K: W = sc (q - 32), |W| <= 4096, has up to 13 bits and enters as Wc, W rounded to a
+// multiple of 16 (8 bits: with x_hi's 11 the sums hardly round), and W - Wc, both exact:
+// four products with the parts of x.  Step n of a half is a window of 32 elements, the
 // lane's 8 a quad of each of its two scale groups.
 template <>
 struct FW<14> {
-  static constexpr int PARTS = 3, ORDER = 2, TU = Fmt<14>::TU, RT = 4, NT = 2;
+  static constexpr int PARTS = 2, ORDER = 2, TU = Fmt<14>::TU, RT = 4, NT = 2;
   static constexpr bool MINS = false;
   Base base;
   int ts, vq, vs, vd;
@@ -245,7 +244,7 @@ struct FW<14> {
     const half2_t sv = __builtin_bit_cast(half2_t, two) + half2_t{(half_t)-1152.f, (half_t)-1152.f};
     const half2_t n1056 = {(half_t)-1056.f, (half_t)-1056.f};
     const half2_t magic = {(half_t)24576.f, (half_t)24576.f};  // its ulp is 16
-    uint32_t wc[4], wl[4], wr[4];
+    uint32_t wc[4], wl[4];
 #pragma unroll
     for (int lh = 0; lh < 2; ++lh) {
       const uint32_t ql = dq[3 * lh + (t & 1)], qh = dq[3 * lh + 2];
@@ -258,12 +257,10 @@ struct FW<14> {
         const half2_t w = __builtin_elementwise_fma(c, sp, magic) - magic;
         wc[2 * lh + o] = __builtin_bit_cast(uint32_t, w);
         wl[2 * lh + o] = pk_fma(c, sp, -w);
-        wr[2 * lh + o] = __builtin_bit_cast(uint32_t, c * sp);
       }
     }
     b[0] = as_h8(wc[0], wc[1], wc[2], wc[3]);
     b[1] = as_h8(wl[0], wl[1], wl[2], wl[3]);
-    b[2] = as_h8(wr[0], wr[1], wr[2], wr[3]);
   }
   static constexpr int Z = 0, HDR = 0;
   __device__ __forceinline__ half4_t mins(int, int) const { return half4_t{}; }
@@ -325,20 +322,20 @@ __global__ __launch_bounds__(256) void gemm_f32_prep_kernel(const float *__restr
 }
 
 // One half unit: 4 steps of 32 elements.  D chains the products of a unit; with
-// PARTS = 3 those of the lo parts and residuals chain in E, and the coarse ones by
+// PARTS = 2 those of the lo parts and residuals chain in E, and the coarse ones by
 // halves of a unit (a long f32 chain at the sum's full size is what rounds most).
 template <int TYPE>
 struct Acc {
   static constexpr int RT = FW<TYPE>::RT, NT = FW<TYPE>::NT, P = FW<TYPE>::PARTS;
-  float4_t acc[RT][NT], D[RT][NT], E[P == 3 ? RT : 1][P == 3 ? NT : 1];
-  float4_t tot[P == 3 ? RT : 1][P == 3 ? NT : 1];  // the sums of each 4 units, added
+  float4_t acc[RT][NT], D[RT][NT], E[P == 2 ? RT : 1][P == 2 ? NT : 1];
+  float4_t tot[P == 2 ? RT : 1][P == 2 ? NT : 1];  // the sums of each 4 units, added
 };
 
 template <int TYPE, int HF>
 __device__ __forceinline__ void half_unit(const FW<TYPE> &w, const unsigned char *stage, int lane,
                                           Acc<TYPE> &a) {
   constexpr int P = FW<TYPE>::PARTS, RT = FW<TYPE>::RT, NT = FW<TYPE>::NT;
-  constexpr int NP = P == 3 ? 3 : 2;  // products
+  constexpr int NP = 2 * P;  // products
   using St = FStage<RT>;
   const float4_t zero = {0.f, 0.f, 0.f, 0.f};
   uint32_t one = kF16Base;  // 1024.0 x 2 in a register: one v_and_or_b32 per masked pair
@@ -360,10 +357,13 @@ __device__ __forceinline__ void half_unit(const FW<TYPE> &w, const unsigned char
       if (!last) w.template operand<HF>(j + 1 < NT ? n : n + 1, j + 1 < NT ? j + 1 : 0, one, bn);
       // the products of one output tile are RT MFMAs apart
 #pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        float4_t &s = P == 3 ? a.E[i % (P == 3 ? RT : 1)][j % (P == 3 ? NT : 1)] : a.D[i][j];
-        s = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], b[P - 1], first ? zero : s, 0, 0, 0);
-      }
+      for (int p = P - 1; p >= 0; --p)
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          float4_t &s = P == 2 ? a.E[i % (P == 2 ? RT : 1)][j % (P == 2 ? NT : 1)] : a.D[i][j];
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], b[p], first && p == P - 1 ? zero : s, 0,
+                                                     0, 0);
+        }
       if (j == NT - 1 && n < 3)  // the fragments' last use: the next step's
 #pragma unroll
         for (int i = 0; i < RT; ++i)
@@ -371,8 +371,8 @@ __device__ __forceinline__ void half_unit(const FW<TYPE> &w, const unsigned char
 #pragma unroll
       for (int i = 0; i < RT; ++i)
         a.D[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            ah[i], b[0], n == 0 && P == 3 ? zero : a.D[i][j], 0, 0, 0);
-      if constexpr (P == 3)
+            ah[i], b[0], n == 0 && P == 2 ? zero : a.D[i][j], 0, 0, 0);
+      if constexpr (P == 2)
 #pragma unroll
         for (int i = 0; i < RT; ++i)
           a.E[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], b[1], a.E[i][j], 0, 0, 0);
@@ -386,11 +386,11 @@ __device__ __forceinline__ void half_unit(const FW<TYPE> &w, const unsigned char
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
         if (j == NT - 1 && n < 3 && (i >= RT * (NP - 1) || i < RT))
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, P == 3 ? 3 : 2, 0);  // two or three VALU
+        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // two VALU
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-  if constexpr (HF == 0 && P != 3) return;
+  if constexpr (HF == 0 && P != 2) return;
   // acc += 2^-e (d D + (Z 32 d) scales . sums - (32 dmin) mins . sums)
 #pragma unroll
   for (int i = 0; i < RT; ++i) {
@@ -413,7 +413,7 @@ __device__ __forceinline__ void half_unit(const FW<TYPE> &w, const unsigned char
           a.acc[i][j][e] = fmaf(f[e], fmaf(d, a.D[i][j][e], fmaf(dz, ss[e], dm * ms[e])),
                                 a.acc[i][j][e]);
         else {  // f d is exact: f is a power of two
-          const float E = HF ? a.E[i % (P == 3 ? RT : 1)][j % (P == 3 ? NT : 1)][e] : 0.f;
+          const float E = HF ? a.E[i % (P == 2 ? RT : 1)][j % (P == 2 ? NT : 1)][e] : 0.f;
           a.acc[i][j][e] = fmaf(f[e] * d, HF ? a.D[i][j][e] + E : a.D[i][j][e], a.acc[i][j][e]);
         }
       }
@@ -457,13 +457,13 @@ __global__ __launch_bounds__(kThr) void gemm_f32_kernel(const unsigned char *__r
   };
 
   Acc<TYPE> a;
-  constexpr int TR = FW<TYPE>::PARTS == 3 ? RT : 1, TN = FW<TYPE>::PARTS == 3 ? NT : 1;
+  constexpr int TR = FW<TYPE>::PARTS == 2 ? RT : 1, TN = FW<TYPE>::PARTS == 2 ? NT : 1;
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       a.acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
-      if (FW<TYPE>::PARTS == 3) a.tot[i % TR][j % TN] = a.acc[i][j];
+      if (FW<TYPE>::PARTS == 2) a.tot[i % TR][j % TN] = a.acc[i][j];
     }
   // The loop body is straight-line: a K half shorter than the other re-reads its last
   // unit and adds zero, and the loads past the last unit re-read it.  With them under
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(kThr) void gemm_f32_kernel(const unsigned char *__r
     w.template load<0>(v);
     w.header(v);
     half_unit<TYPE, 1>(w, s1, lane, a);
-    if (FW<TYPE>::PARTS == 3 && ((i & 3) == 3 || i == h0 - 1)) {
+    if (FW<TYPE>::PARTS == 2 && ((i & 3) == 3 || i == h0 - 1)) {
 #pragma unroll
       for (int p = 0; p < RT; ++p)
 #pragma unroll

@@ -169,6 +169,25 @@ def test_batched_decode_random_blocks(pkg, ref, t, xdt):
             outs.append(y)
 
 
+def test_f32_gemm_q6_k_weights_are_exact(pkg):
+    """Every part of an activation meets the exact Q6_K integer: with W = 127 * 31 = 3937 (12
+    bits, the middle of two f16 values) and pairs x = 1 + e, -1 with e below an f16 step, the
+    leading parts cancel and the result is 3937 sum e.  Bound: the sums' own rounding, 64
+    chained f32 additions of terms of one sign."""
+    n, k, m = 70, 512, 40
+    raw = np.full((n, k // 256, 210), 0xFF, np.uint8)
+    raw[..., 192:208] = 127
+    raw[..., 208:210] = np.array([1.0], np.float16).view(np.uint8)
+    w = pkg.repack_gguf_for_gpu(14, raw.reshape(-1), n, k)
+    e = np.random.default_rng(2).integers(1, 1 << 11, (m, k // 2)) * 2.0 ** -23
+    x = np.stack([1 + e, -np.ones_like(e)], axis=2).reshape(m, k).astype(np.float32)
+    want = 3937.0 * e.sum(1)
+    for rows in (m, 32):
+        y = pkg.qlinear(torch.from_numpy(x[:rows]).cuda(), w).cpu().numpy().astype(np.float64)
+        err = np.abs(y - want[:rows, None]) / want[:rows, None]
+        assert err.max() <= 64 * 2.0 ** -24, (rows, err.max())
+
+
 @pytest.mark.parametrize("t", [13, 2, 6, 20, 23])
 @pytest.mark.parametrize("xdt", [np.float32, np.float16])
 def test_batched_decode_more_types(pkg, ref, t, xdt):
