@@ -25,8 +25,8 @@
 //   operand 4 row tiles and both parts.  The operand is the exact f16 integer
 //   sc (q - Z) (Q6_K: the sum of two); the codes come straight from memory.
 // Measured against the 32-row passes, whole call: Q4_K 128 x 28672 x 4096
-// 146 -> 77 us, Q6_K 387 x 4096 x 14336 313 -> 188, Q5_K 200 x 14336 x 4096 415 -> 120,
-// Q6_K 500 x 14336 x 4096 424 -> 232, Q4_K 40 x 4096 x 4096 26 -> 22; the error against
+// 146 -> 77 us, Q6_K 387 x 4096 x 14336 313 -> 187, Q5_K 200 x 14336 x 4096 415 -> 117,
+// Q6_K 500 x 14336 x 4096 424 -> 229, Q4_K 40 x 4096 x 4096 26 -> 22; the error against
 // float64 fell (Q4_K 3.0e-7 -> 1.9e-7, Q6_K 1.25e-7 -> 1.09e-7).  What bounds it: the
 // vector work of the operands (35 of the 78 us of the first, by leaving it out) and
 // the MFMAs beside it (28 us at their full rate) hardly overlap on two waves per SIMD.
@@ -66,14 +66,14 @@ struct Base {
   uint32_t lo, hi;
   int bytes;
   __device__ __forceinline__ rsrc_t rs() const {
-    const uint64_t p = (uint32_t)__builtin_amdgcn_readfirstlane(lo) |
-                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(hi) << 32;
-    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, __builtin_amdgcn_readfirstlane(bytes),
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(lo | (uint64_t)hi << 32), 0, bytes,
                                              0x00020000);
   }
 };
 __device__ __forceinline__ Base make_base(const void *p, int bytes) {
-  return Base{(uint32_t)(uintptr_t)p, (uint32_t)((uintptr_t)p >> 32), bytes};
+  return Base{(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p),
+              (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)((uintptr_t)p >> 32)),
+              __builtin_amdgcn_readfirstlane(bytes)};
 }
 __device__ __forceinline__ uint32_t pk_fma(half2_t a, half2_t b, half2_t c) {
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(a, b, c));
@@ -469,6 +469,11 @@ __global__ __launch_bounds__(kThr) void gemm_f32_kernel(const unsigned char *__r
   // unit and adds zero, and the loads past the last unit re-read it.  With them under
   // a condition the memory counter's waits assume that they were not issued, and each
   // half unit would wait for its own prefetch.
+  // The unit's headers are read before its second half's stage is requested: after that
+  // the compiler cannot tell them from the stage and waits for it.  (At a unit's end, where
+  // the next stage has been in flight for half a unit, the sums' reads wait for it in Q4_K
+  // and Q5_K; Q4_K reloads three of five spilled registers there.)  14336 x 4096, Q5_K, 128
+  // rows 64.9 -> 62.0 us, 28672 x 4096, Q4_K, 128 rows 78.8 -> 76.8.
   const int ul = min(ua + un, u0 + max(cnt, 1)) - 1;
   stage(min(u0, ul), 0, s0);
   w.template load<0>(min(u0, ul));
@@ -480,9 +485,9 @@ __global__ __launch_bounds__(kThr) void gemm_f32_kernel(const unsigned char *__r
     const int u = min(u0 + i, ul), v = min(u0 + i + 1, ul);
     const bool act = i < cnt;
     __syncthreads();  // the first half's stage has arrived, the second's is free
+    w.begin(act);
     stage(u, 1, s1);
     w.template load<1>(u);
-    w.begin(act);
     half_unit<TYPE, 0>(w, s0, lane, a);
     __syncthreads();
     stage(v, 0, s0);
