@@ -539,9 +539,13 @@ struct F32Plan {
   int rb, cb, nu, sp, kunits;
   int64_t img, part;  // floats
 };
-// K splits by estimated time: rounds of 256 workgroups (one per CU, MI355X), each
-// 2.3 us a unit and 4 us besides; splitting costs a second launch and the partial
-// sums' write and read.
+// K splits by estimated time: rounds of 256 workgroups (one per CU, MI355X), each the
+// type's microseconds a unit and K half, 15% more with every CU at work; splitting costs a
+// second launch and the partial sums' write and read.  Fitted to 1, 2, 3, 4, 6, 8, 12 and 16
+// splits of 11 weights (1024 x 512 to 32000 x 2048 and 4096 x 14336) at 33 to 511 rows, 5 to
+// 7% rms; the split chosen is within 0.3% of the best on average and 5% at worst.  In us,
+// 1 split / the one chosen: Q4_K 14336 x 4096, 128 rows 68.5 / 48.5 (2); 4096^2, 387 rows
+// 70.5 / 50.0 (2); 1024^2, 33 rows 22.6 / 17.7 (2); Q6_K 4096 x 14336, 387 rows 195 (1; 2: 200).
 template <int TYPE>
 F32Plan plan(int64_t n, int64_t k, int64_t m) {
   F32Plan p;
@@ -554,8 +558,10 @@ F32Plan plan(int64_t n, int64_t k, int64_t m) {
   for (int s = 1; s <= 16 && s <= p.nu; ++s) {
     const int ku = (p.nu + s - 1) / s;
     if ((p.nu + ku - 1) / ku != s) continue;  // an empty last split
-    const int64_t rounds = ((int64_t)p.rb * p.cb * s + 255) / 256;
-    const double us = rounds * (2.3 * ((ku + 1) / 2) + 4) + (s > 1 ? 4 + s * m * n * 8 / 4e6 : 0);
+    const int64_t wgs = (int64_t)p.rb * p.cb * s, rounds = (wgs + 255) / 256;
+    const double unit = TYPE == 12 ? 7.0 : TYPE == 13 ? 6.3 : 5.8;
+    const double us = rounds * ((ku + 1) / 2) * unit * (1 + 0.15 * (wgs < 256 ? wgs / 256.0 : 1)) +
+                      (s > 1 ? 1.8 + s * m * n * 8 / 3.9e6 : 0);
     if (s == 1 || us < best) {
       best = us;
       p.sp = s;
@@ -590,8 +596,17 @@ hipError_t launch(const float *x, int64_t ldx, const uint8_t *W, int64_t n, int6
 
 }  // namespace
 
-// From 33 rows to the row count from which f32 batches take the fp16 GEMM; a
-// weight's row tile keeps 32-bit byte offsets.
+// From 33 rows to the row count from which f32 batches take the fp16 GEMM, at any size; a
+// weight's row tile keeps 32-bit byte offsets.  Graph replays in us, 32-row passes / here:
+//   rows               33           64           128          511
+//   Q4_K 256 x 512     20.9 / 15.4  29.0 / 16.2  57.4 / 16.6  228 / 16.9
+//        1024^2        18.9 / 17.6  29.4 / 18.6  58.2 / 19.1  232 / 22.4
+//        14336 x 4096  30.4 / 30.5  43.5 / 33.3  86.3 / 48.5  337 / 142
+//   Q5_K 1024^2        15.7 / 15.6  22.0 / 16.6  43.7 / 17.0  173 / 20.9
+//   Q6_K 256 x 512     21.5 / 12.3  34.3 / 12.9  68.4 / 13.2  272 / 13.8
+//        14336 x 4096  37.4 / 39.1  55.4 / 41.0  109 / 64     433 / 236
+// 33 rows are one 32-row pass and the one-row kernel there, and the only count where the
+// passes are level, by up to 4%, at 58 million weights (256 x 14336 also, 26.0 / 26.4).
 bool gemm_f32_serves(int type, int x_type, int64_t n, int64_t k, int64_t m) {
   return x_type == 0 && m > 32 && m < GGUF_HIP_F32_GEMM_MIN_M && (type == 12 || type == 13 || type == 14) && k % 256 == 0 &&
          k <= ((int64_t)1 << 24);
