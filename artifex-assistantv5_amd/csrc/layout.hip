@@ -804,15 +804,17 @@ __global__ __launch_bounds__(256) void dequant_raw_kernel(const uint8_t *__restr
 // [0, n_rows) reads nothing and writes a row of NaN, so a bad token id is visible in the
 // output instead of faulting.
 //
-// Rows of 4096 values, direct / through LDS, in us: Q4_K 1 row 4.4 / 3.7, 64 10.7 / 6.4,
-// 1900 77 / 9.4; Q6_K 1 row 6.6 / 6.8, 8 17.9 / 12.4, 1900 55 / 18.6; Q3_K (and Q2_K) 1900
-// 13.6 / 14.0; the others alike, Q8_0: 64 rows 3.4 / 3.8, 1024 9.6 /
-// 6.3, 1900 15.4 / 8.4 (the stores' pieces merge in L2 until the output outgrows it;
-// before that the detour is latency); Q5_K 1024 9.0 / 9.7, 1900 14.2 / 12.3.
+// Direct / through LDS, in us.  Q4_K: 1 row of 512 3.1 / 3.4, of 2048 3.6 / 3.7, of 4096
+// 4.4 / 3.7, 8 rows of 512 4.5 / 3.9, 4 of 1024 4.5 / 3.9, 1900 of 4096 77 / 9.4.  Q6_K: 32 rows
+// of 512 10.6 / 12.7, 8 of 2048 9.9 / 12.3, 32 of 1024 19.4 / 12.5, 8 of 4096 17.9 / 12.4, 1900 of
+// 4096 55 / 18.6.  Q3_K (and Q2_K) 1900 of 4096 13.6 / 14.0.  The others alike, Q8_0: 64 of
+// 4096 3.4 / 3.8, 512 of 8192 9.8 / 6.5, 4096 of 1024 9.8 / 6.5, 1900 of 4096 15.4 / 8.4 (the
+// stores' pieces merge in L2 until the output outgrows it; before that the detour is
+// latency); Q5_K 1024 of 4096 9.0 / 9.7, 512 of 14336 13.7 / 12.5, 1900 of 4096 14.2 / 12.3.
 template <int TYPE>
-constexpr bool get_rows_lds(int64_t n_ids, int64_t values) {
-  return TYPE == 12 || (TYPE == 14 && n_ids >= 8) ||
-         (TYPE != 14 && TYPE != 10 && TYPE != 11 && values >= (int64_t)(TYPE == 13 ? 3 : 2) << 21);
+constexpr bool get_rows_lds(int64_t values) {
+  return TYPE != 10 && TYPE != 11 &&
+         values >= (TYPE == 12 ? 4096 : TYPE == 14 ? 32768 : (int64_t)(TYPE == 13 ? 3 : 2) << 21);
 }
 template <int TYPE, bool LDS>
 constexpr int get_rows_threads() { return LDS && RawPiece<TYPE>::VALUES > 64 ? 128 : 256; }
@@ -901,7 +903,7 @@ static void get_rows_type(const uint8_t *raw, int64_t n_rows, int64_t k, const i
                        dim3((unsigned)((threads + NT - 1) / NT)), dim3(NT), 0, s, raw, n_rows, upr,
                        ids, n_ids, out, ldo);
   };
-  if (get_rows_lds<TYPE>(n_ids, n_ids * k))
+  if (get_rows_lds<TYPE>(n_ids * k))
     launch(std::true_type());
   else
     launch(std::false_type());

@@ -46,6 +46,17 @@ def test_get_rows_bit_exact(ref, t):
     assert np.isnan(o[1:, :k]).all() and (o[:, k:] == 0).all()
 
 
+@pytest.mark.parametrize("t,m", [(12, 1), (12, 7), (12, 8), (14, 8), (14, 63), (14, 64)])
+def test_get_rows_few_narrow_rows(ref, t, m):
+    """Both sides of the size from which the rows go through LDS, rows of 512 values."""
+    n, k = 9, 512
+    raw = pkg.quantize.quantize(pkg.quantize.synthetic_weight(n, k, seed=t, std=1.0), t)
+    table = pkg.QuantEmbedding(torch.from_numpy(raw).cuda(), t, n, k)
+    ids = np.random.default_rng(m).integers(0, n, m)
+    o = table.gather(torch.from_numpy(ids).cuda()).cpu().numpy()
+    assert ref.same_bits(o, ref.dequant_rows(t, raw, n, k)[ids])
+
+
 @pytest.mark.parametrize("t", [2, 11, 12, 14, 23])
 def test_get_rows_many(ref, t):
     """Rows that straddle workgroups, a last workgroup that is not full, strided output rows
