@@ -46,8 +46,7 @@ bool traits(int t, int *block, int *size) {
 }
 
 // The grid-codebook IQ types.  Their decode variant needs a workspace only
-// beyond K = kIqOneShotMaxK (the one-shot kernel's staging limit).
-constexpr int64_t kIqOneShotMaxK = 16384;
+// beyond K = GGUF_HIP_ONE_SHOT_MAX_K (the one-shot kernel's staging limit).
 bool grid_type(int t) {
   return t == GGUF_HIP_IQ2_XXS || t == GGUF_HIP_IQ2_XS || t == GGUF_HIP_IQ2_S ||
          t == GGUF_HIP_IQ3_XXS || t == GGUF_HIP_IQ3_S || t == GGUF_HIP_IQ1_M;
@@ -251,7 +250,7 @@ int gguf_hip_matmul_ws(const void *x, int x_type, int64_t ldx, const void *tiles
   // grid types: up to K = 16384 the decode variant runs without a workspace
   // (the one-shot kernel, once per row when the workspace is missing); beyond
   // it only the batched kernel serves them, and that needs one
-  if (grid_type(ggml_type) && variant == GGUF_HIP_VARIANT_DECODE && k > kIqOneShotMaxK) {
+  if (grid_type(ggml_type) && variant == GGUF_HIP_VARIANT_DECODE && k > GGUF_HIP_ONE_SHOT_MAX_K) {
     const int64_t need = 4 * gguf::launch_decode_work(ggml_type, x_type, n, k, m);
     if (need > 0 && (!work || work_bytes < need))
       return fail(GGUF_HIP_ERR_SHAPE,
@@ -293,7 +292,7 @@ int64_t gguf_hip_matmul_workspace(int ggml_type, int x_type, int64_t n, int64_t 
   if (n == 0 || m == 0) return 0;
   // the larger of the decode path's and the GEMM's (AUTO may take either)
   // (M = 1: the one-shot kernel needs none; grid types above K = 16384 still do)
-  const int64_t dec = (m < 2 && (!grid_type(ggml_type) || k <= kIqOneShotMaxK))
+  const int64_t dec = (m < 2 && (!grid_type(ggml_type) || k <= GGUF_HIP_ONE_SHOT_MAX_K))
                           ? 0 : gguf::launch_decode_work(ggml_type, x_type, n, k, m);
   int64_t gem = m > 32 ? gguf::launch_gemm_work(ggml_type, x_type, n, k, m) : 0;
   if (gem > 0) gem += gguf::kWsPrefix / 4;  // the GEMM's partial sums follow the counter prefix
@@ -449,8 +448,9 @@ int gguf_hip_matmul_fused(const float *x, const void *tiles, int ggml_type, int6
   if (epilogue == GGUF_HIP_EPILOGUE_SWIGLU && n % 32)
     return fail(GGUF_HIP_ERR_SHAPE, "[gguf-hip] SwiGLU epilogue: N %% 32 != 0");
   if (n < 0 || n > ((int64_t)1 << 30)) return fail(GGUF_HIP_ERR_SHAPE, "[gguf-hip] bad N");
-  if (k > 16384)
-    return fail(GGUF_HIP_ERR_SHAPE, "[gguf-hip] fused matmul: K=%lld above 16384", (long long)k);
+  if (k > GGUF_HIP_ONE_SHOT_MAX_K)
+    return fail(GGUF_HIP_ERR_SHAPE, "[gguf-hip] fused matmul: K=%lld above %d", (long long)k,
+                GGUF_HIP_ONE_SHOT_MAX_K);
   if (k % 16) return fail(GGUF_HIP_ERR_SHAPE, "[gguf-hip] fused matmul: K %% 16 != 0");
   if (prologue == GGUF_HIP_PROLOGUE_RMSNORM && !(eps >= 0.0f))
     return fail(GGUF_HIP_ERR_SHAPE, "[gguf-hip] rmsnorm: eps must be >= 0");

@@ -38,6 +38,7 @@
 
 #include "common.hpp"
 #include "decode_types.hpp"
+#include "gguf_hip.h"
 #include "iq.hpp"
 #include "iq_ops.hpp"
 
@@ -1790,7 +1791,7 @@ hipError_t launch_m1(const XT *x, const uint8_t *W, int N, int K, float *y, cons
   constexpr int UE = Fmt<TYPE>::UE, GS = Dec<TYPE>::GS;
   constexpr int PARTS = sizeof(XT) == 4 ? 2 : 1;
   const int ntiles = (N + 15) / 16, nu = K / UE;
-  if (K > 16384) return hipErrorNotSupported;
+  if (K > GGUF_HIP_ONE_SHOT_MAX_K) return hipErrorNotSupported;
   const bool long_k = K > 4096;
   const int umax = m1_umax<TYPE>(long_k || (PRO != 0 && GGUF_M1_PRO_TIGHT));
   // K split: units per wave within the budget, and at least ~1024 waves when

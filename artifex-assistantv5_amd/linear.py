@@ -364,8 +364,8 @@ def dispatch_matmul_gguf(a: torch.Tensor, gg: GGUFWeight, c: torch.Tensor, M: in
     dev = gg.device
     x_type = _X_TYPES[a.dtype]
     # the split-K paths' workspace (activation image, partial sums of the K slices)
-    # one row of up to 16384 elements takes the one-shot kernel, which needs no workspace
-    need = 0 if M == 1 and K <= 16384 else \
+    # one row takes the one-shot kernel, which needs none, up to its limit
+    need = 0 if M == 1 and K <= _native.ONE_SHOT_MAX_K else \
         _native.check(lib.gguf_hip_matmul_workspace(gg.ggml_type, x_type, N, K, M), lib)
     work = matmul_workspace(dev, need) if need > 0 else None
     # the device guard costs as much as the launch; it is needed on another device only

@@ -102,6 +102,7 @@ extern "C" {
                                      activations staged in LDS (prefill); f32 activation
                                      rows are scaled by a power of two each first */
 #define GGUF_HIP_DECODE_MAX_M 32
+#define GGUF_HIP_ONE_SHOT_MAX_K 16384 /* one row of up to this K needs no workspace */
 #define GGUF_HIP_F32_GEMM_MIN_M 512
 
 /* ABI version of the loaded library (GGUF_HIP_ABI_VERSION). */

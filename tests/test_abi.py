@@ -72,6 +72,19 @@ def test_constants_match_header(native):
             d["GGUF_HIP_IQ2_S"], d["GGUF_HIP_IQ1_M"]) == (16, 17, 18, 21, 22, 29)
 
 
+def test_one_row_needs_no_workspace_up_to_the_limit(lib, native, pkg):
+    """The host asks for no workspace for one row of up to ONE_SHOT_MAX_K elements."""
+    limit = native.ONE_SHOT_MAX_K
+    assert _defines()["GGUF_HIP_ONE_SHOT_MAX_K"] == limit
+    for t in (2, 6, 8, 10, 11, 12, 13, 14, 16, 17, 18, 20, 21, 22, 23, 29):
+        for x_type in (0, 1):
+            for n in (1, 4096, 151936):
+                for k in (256, 4096, limit - 256, limit):
+                    assert lib.gguf_hip_matmul_workspace(t, x_type, n, k, 1) == 0, (t, n, k)
+    for t in (16, 17, 18, 21, 22, 29):
+        assert lib.gguf_hip_matmul_workspace(t, 0, 4096, limit + 256, 1) > 0
+
+
 def test_grid_types_contract(lib, native):
     """IQ2_XXS .. IQ1_M: no workspace needed for the decode variant up to
     K = 16384 (M = 1 asks for none, M >= 2 for an optional one); beyond it a
