@@ -446,10 +446,11 @@ __global__ __launch_bounds__(kGlueThreads) void attention_prefill_kernel(
   __shared__ __align__(16) float vt[HD * VLD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, g4 = lane >> 4;  // MFMA column (row of the block), k group
-  // the workgroups in launch order: KV head fastest, the last rows first
-  const int64_t b = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-  const int grp = nh / nkv, kvh = (int)(b % nkv);
-  const int64_t m = ((int64_t)gridDim.x - 1 - b / nkv) * kPfRows + col;
+  // the workgroups in launch order: KV head fastest, the last rows first (the number of a
+  // workgroup fits 32 bits: each has 16 rows of K and V of at least 64 values)
+  const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x, rb = b / (uint32_t)nkv;
+  const int grp = nh / nkv, kvh = (int)(b - rb * (uint32_t)nkv);
+  const int64_t m = (int64_t)(gridDim.x - 1 - rb) * kPfRows + col;
   int my = -1;  // the row's position; -1: attends to nothing, not written
   if (m < M) {
     const int64_t p = pos[m];
