@@ -1376,7 +1376,7 @@ template <int TYPE, typename XT>
 int64_t mb_work_floats(int M, int N, int K) {
   if (M < 2) return 0;
   if constexpr (TYPE != 10 && TYPE != 11)  // the batched kernel (decode_mk.hpp)
-    if (mk_takes<TYPE>(M, N, K)) return (int64_t)((mk_work_bytes<TYPE, XT>(M, N, K) + 3) / 4);
+    if (mk_takes<TYPE>(M, N, K, sizeof(XT) == 2)) return (int64_t)((mk_work_bytes<TYPE, XT>(M, N, K) + 3) / 4);
   int us, nsl;
   mb_plan<TYPE, XT>(M, N, K, &us, &nsl);
   return nsl > 1 ? kWsPrefix / 4 + (int64_t)nsl * M * N : 0;
@@ -1898,7 +1898,7 @@ hipError_t launch_m(const XT *x, int64_t ldx, const uint8_t *W, int N, int K, fl
     if (e != hipErrorNotSupported) return e;
   }
   if constexpr (TYPE != 10 && TYPE != 11) {  // the batched kernel (decode_mk.hpp)
-    const hipError_t e = mk_takes<TYPE>(M, N, K)
+    const hipError_t e = mk_takes<TYPE>(M, N, K, sizeof(XT) == 2)
                              ? launch_mk<TYPE, XT>(x, ldx, W, N, K, y, ldy, M, work, work_floats, s)
                              : hipErrorNotSupported;
     if (e != hipErrorNotSupported) return e;

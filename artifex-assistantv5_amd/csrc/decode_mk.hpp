@@ -949,24 +949,29 @@ size_t mk_work_bytes(int M, int N, int K) {
 //           (f16 12.1 / 12.8); 14336 x 1024: 20.0 / 10.6; 4096 x 1024: 7.8 / 10.5;
 //           512 x 8192: 15.7 / 13.1
 //   IQ4_XS  8192 x 4096: 17.3 / 13.9; 4096^2 13.9 / 13.0, f16 12.0 / 12.9;
-//           14336 x 1024: 19.8 / 10.7; 512 x 8192: 15.7 / 13.6, but M = 32 18.7 / 20.9
+//           14336 x 1024: 19.8 / 10.7; 512 x 8192: M = 8 16.0 / 14.0, 12 14.7 / 16.2, 16
+//           16.3 / 16.1, 32 18.7 / 20.9, f16 M = 8 15.5 / 14.2, 16 15.7 / 14.5
 //   Q5_0 (Q4_0 and IQ4_NL alike)  14336 x 4096: M = 2 20.7 / 15.5, 32 54.7 / 27.9;
 //           8192 x 4096: f16 12.7 / 13.6; narrow weights, where mb_kernel has few
 //           workgroups and many slices: 1000 x 1024 13.9 / 10.7 (M = 32 15.7 / 20.3),
-//           1024 x 4096 15.4 / 13.1, 512 x 14336 34.4 / 16.2; 4096 x 2048 9.4 / 12.8
+//           1024 x 4096 15.4 / 13.1, 512 x 14336 34.4 / 16.2; 4096 x 2048 9.4 / 12.8;
+//           1000 x 3072 M = 8 14.5 / 13.4, 12 14.3 / 15.5 (IQ4_NL 14.4 / 14.9, but Q4_0
+//           14.8 / 12.9), f16 M = 12 14.0 / 13.6; 1024^2 M = 12 15.4 / 13.2
 template <int TYPE>
-bool mk_takes(int M, int N, int K) {
+bool mk_takes(int M, int N, int K, bool f16) {
   if (TYPE == 10 || TYPE == 11 || K % 256 != 0) return false;
   const int64_t units = (int64_t)((N + 15) / 16) * (K / 256);
+  const bool one = M <= (f16 ? 16 : 8);  // one activation tile
   if (TYPE == 13)
     return M > 1 && (K >= 8192 || units >= 6144 || (units >= 2048 && (M > 16 || K >= 4096)) ||
                      (units >= 3072 && K <= 1024));
   if (TYPE == 23)
-    return M > 1 && (units >= 6144 || (K >= 8192 && (M <= 16 || units >= 1536)) ||
+    return M > 1 && (units >= 6144 || (K >= 8192 && (one || units >= 1536)) ||
                      (units >= 3072 && K <= 1024));
   if (TYPE == 2 || TYPE == 6 || TYPE == 20)
     return M > 1 && ((units >= 12288 && K >= 4096) ||
-                     (N <= 1024 && K >= 1024 && (M <= 16 || K >= 4096)));
+                     (N <= 1024 && K >= 1024 &&
+                      (one || K >= 4096 || (M <= 16 && (TYPE == 2 || K <= 1024)))));
   return true;
 }
 

@@ -220,6 +220,23 @@ def test_batched_decode_more_types(pkg, ref, t, xdt):
             assert met["finite"] and met["elemwise"] <= DECODE_TOL, ((t, m, n, k, use_ws), met)
 
 
+@pytest.mark.parametrize("t,n,k", [(6, 300, 3072), (20, 300, 3072), (2, 300, 3072), (6, 40, 1024),
+                                   (23, 64, 8192)])
+@pytest.mark.parametrize("xdt", [np.float32, np.float16])
+def test_batched_decode_narrow_weights(pkg, ref, t, n, k, xdt):
+    """Narrow weights where the kernel goes by the activation tiles: one tile (8 f32 or 16
+    f16 rows) and one row more, with the workspace that the host asks for."""
+    raw = tile_model.random_blocks(t, n, k, seed=t + n, specials=False)
+    w = pkg.repack_gguf_for_gpu(t, raw, n, k)
+    wdeq = ref.dequant_rows(t, raw, n, k)
+    for m in (8, 9, 16, 17):
+        x = np.random.default_rng(m).standard_normal((m, k)).astype(xdt)
+        y = pkg.qlinear(torch.from_numpy(x).cuda(), w, variant=DECODE).cpu().numpy()
+        x64 = x.astype(np.float64)
+        met = ref.parity_metrics(y, ref.matmul_bt(x64, wdeq), ref.matmul_bt_abs(x64, wdeq))
+        assert met["finite"] and met["elemwise"] <= DECODE_TOL, ((t, m, n, k), met)
+
+
 @pytest.mark.parametrize("t", [8, 12, 14, 16])
 @pytest.mark.parametrize("m", [2, 16, 17])
 def test_batched_decode_short_k(pkg, ref, t, m):
