@@ -95,7 +95,8 @@ def attention_decode(qkv: torch.Tensor, pos: torch.Tensor, cos: torch.Tensor, si
                      n_heads: int, n_kv_heads: int, head_dim: int,
                      work: torch.Tensor) -> torch.Tensor | None:
     """RoPE + KV append at slot ``pos`` (device int64 [1]) + causal GQA attention.
-    ``out=None`` writes only the partial-softmax records into ``work``, for
+    ``out=None`` writes the partial-softmax records into ``work`` (beyond 2048 slots a
+    second launch merges them there), for
     ``matmul_attn_merge`` to merge inside the output projection.  Caches are
     ``[n_kv_heads, max_seq, head_dim]``, cos / sin ``[max_seq, head_dim / 2]``."""
     if k_cache.dim() < 2:
